@@ -12,7 +12,7 @@ the state resident in HBM.  One JSON line is printed.
 The roofline block times the dominant kernel with HIP events recorded on
 the context's stream during the timed region and divides its algorithmic
 bytes per launch (mesh/state bytes it must read, intermediates excluded) by
-the average launch time: the viscous apply k_diff_apply when the viscous
+the average launch time: the viscous apply k_visc_apply when the viscous
 terms are on (``roofline_node_sweep`` then gives the node sweep's), the node
 sweep k_node_flux otherwise.  The CPU baseline times the oracle on the host
 cores (one process per core of the GPU's CPU share) on bounded samples of the
@@ -46,13 +46,12 @@ def algorithmic_bytes(C, V, SF, SE, second_order):
 
 
 def diff_apply_bytes(C, V, SF, SE, block_doubles):
-    """Bytes the viscous apply must move per launch: the packed per-vertex
-    blocks (N^-1 S, S~^T N^-1 S, their right-hand sides and the heat-system
-    counterparts, built once per mesh), each sub-face's unit normal, area and
-    left cell, each slot's cell, sub-element id, sub-element volume, offset
-    and sub-face list (three entries for a prism corner), each cell's state
-    once, the vertex offsets, and the 18-double slot rows it writes."""
-    return block_doubles * 8 + SF * 36 + SE * (4 + 4 + 8 + 4 + 12) + C * 40 + V * 16 + SE * 144
+    """Bytes the viscous apply must move per launch: the packed inverses of the
+    vertices' nodal systems (built once per mesh), each sub-face's unit normal,
+    area and place, each slot's cell, face codes and inverse sub-element volume,
+    each cell's state once, the vertex offsets, and the four-double slot rows it
+    writes."""
+    return block_doubles * 8 + SF * 33 + SE * (4 + 4 + 8) + C * 40 + V * 16 + SE * 32
 
 
 def stage_bytes_m1(C, V, SF, SE):
@@ -371,8 +370,8 @@ def main():
         dbytes = diff_apply_bytes(C, V, SF, SE, s.count("diff_block_doubles"))
         dach = dbytes / (da["us_avg"] * 1e-6) / 1e9
         roofline = {
-            "bound": "hbm", "kernel": "k_diff_apply", "achieved": dach, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-            "frac": dach / HBM_PEAK_GBS, "traffic": read_traffic(f"k_diff_apply_{tag}"),
+            "bound": "hbm", "kernel": "k_visc_apply", "achieved": dach, "peak": HBM_PEAK_GBS, "unit": "GB/s",
+            "frac": dach / HBM_PEAK_GBS, "traffic": read_traffic(f"k_visc_apply_{tag}"),
             "algorithmic_bytes_per_launch": dbytes, "us_per_launch": da["us_avg"], "launches": da["launches"],
         }
         extra = {"roofline_node_sweep": node_roof}

@@ -135,19 +135,20 @@ struct subfv_ctx {
   double *W = nullptr;    // [C][6] primitives and sound speed of the state a residual works on
   bool ngp_ready = false;
   double *blk = nullptr;
-  // viscous terms: per-vertex precomputed blocks (once per mesh with a
-  // constant viscosity, every residual with Sutherland's law)
+  // viscous terms: the inverses of each vertex's nodal systems (once per mesh
+  // with a constant viscosity, every residual with Sutherland's law)
   bool diff_on = false, diff_ready = false;
   DiffParams dparams{};
-  long *doff = nullptr;
+  uint64_t *doff = nullptr;
   double *pre = nullptr, *PD = nullptr, *rdiff = nullptr;
-  uint32_t *dssf = nullptr;  // [SE] node-sorted slot -> its sub-element's vertex-local sub-faces, packed
-  double *dsvol = nullptr;   // [SE] node-sorted slot -> sub-element volume
+  uint32_t *dscode = nullptr;  // [SE] node-sorted slot -> its sub-element's faces, packed
+  uint8_t *dfpos = nullptr;    // [SF] a sub-face's place among its vertex's faces
+  double *dsivol = nullptr;    // [SE] node-sorted slot -> 1 / sub-element volume
+  double *dblk = nullptr;      // [C][kDiffBlk] the cells' viscous blocks
   double *mu_cell = nullptr, *mu_blk = nullptr;  // Sutherland: [C] viscosities; block minima + mu0corr
-  int diff_fm = 0, diff_em = 0;  // setup LDS extents: 3 * max sub-faces, 3 * max sub-elements of a vertex
-  bool diff_large = false;        // a vertex beyond the small size class: large-class kernels
-  double *dws = nullptr;          // large class: the setup's workspace, kDiffWsBlocks blocks
-  long pre_n = 0;  // doubles in the packed viscous blocks
+  int diff_cls = 0;  // DiffClass of the mesh
+  int diff_nim = 0, diff_nfm = 0, diff_nsm = 0, diff_lmat = 0;  // a vertex's largest sizes (DiffArgs)
+  long pre_n = 0;  // doubles in the packed inverses
   int *derr = nullptr;  // [2]: error bits of the path, failed check_mesh cells
   StepState *st = nullptr;
   double host_t = 0.0;
@@ -245,10 +246,11 @@ void free_mesh(subfv_ctx *c) {
   c->NG = c->VMM = c->G = c->vp = c->diag = c->blk = c->NGP = c->W = nullptr;
   c->ngp_ready = false;
   c->doff = nullptr;
-  c->pre = c->PD = c->rdiff = c->dsvol = nullptr;
-  c->dssf = nullptr;
+  c->pre = c->PD = c->rdiff = c->dsivol = nullptr;
+  c->dscode = nullptr;
+  c->dfpos = nullptr;
+  c->dblk = nullptr;
   c->mu_cell = c->mu_blk = nullptr;
-  c->dws = nullptr;
   c->diff_ready = false;
 }
 
@@ -630,8 +632,18 @@ int launch_grad(subfv_ctx *c, const double *U, int method, const double *W = nul
   return 0;
 }
 
+template <int DIAG>
+void launch_update_d(subfv_ctx *c, const UpdateArgs &u) {
+  dim3 g(nblk(c->dm.C, kCellThreads)), b(kCellThreads);
+  hipLaunchKernelGGL(k_update<DIAG>, g, b, 0, c->stream, u);
+  hipLaunchKernelGGL(k_finalize_omega, dim3(1), b, 0, c->stream, (const double *)c->blk, (int)g.x, c->st, u.advance_t);
+  hipLaunchKernelGGL(k_update_fixup<DIAG>, g, b, 0, c->stream, u);
+}
+
+// Ud: the state of the residual whose viscous terms enter (the stages of a run);
+// null: the diag array as it stands, its rhs already in rhs (the single update)
 int launch_update(subfv_ctx *c, const double *U, const double *U0, double *Uout, double a1, double a2, double w0,
-                  double w1, int flux_limit, int advance_t, bool with_diff = false) {
+                  double w1, int flux_limit, int advance_t, const double *Ud = nullptr) {
   UpdateArgs u;
   u.m = c->dm;
   u.U = U;
@@ -641,7 +653,10 @@ int launch_update(subfv_ctx *c, const double *U, const double *U0, double *Uout,
   u.rhs2 = c->rhs2;
   u.sl = c->sl;
   u.diag = c->diff_on ? c->diag : nullptr;
-  u.rdiff = (c->diff_on && with_diff) ? c->rdiff : nullptr;
+  u.rdiff = (c->diff_on && Ud) ? c->rdiff : nullptr;
+  u.Ud = Ud;
+  u.dblk = c->dblk;
+  u.cv = c->dparams.cv;
   u.blk = c->blk;
   u.st = c->st;
   u.a1 = a1;
@@ -650,106 +665,109 @@ int launch_update(subfv_ctx *c, const double *U, const double *U0, double *Uout,
   u.w1 = w1;
   u.flux_limit = flux_limit;
   u.advance_t = advance_t;
-  dim3 g(nblk(c->dm.C, kCellThreads)), b(kCellThreads);
   Prof pf(c, "update");
-  if (u.diag) {
-    hipLaunchKernelGGL(k_update<true>, g, b, 0, c->stream, u);
-    hipLaunchKernelGGL(k_finalize_omega, dim3(1), b, 0, c->stream, (const double *)c->blk, (int)g.x, c->st, advance_t);
-    hipLaunchKernelGGL(k_update_fixup<true>, g, b, 0, c->stream, u);
-  } else {
-    hipLaunchKernelGGL(k_update<false>, g, b, 0, c->stream, u);
-    hipLaunchKernelGGL(k_finalize_omega, dim3(1), b, 0, c->stream, (const double *)c->blk, (int)g.x, c->st, advance_t);
-    hipLaunchKernelGGL(k_update_fixup<false>, g, b, 0, c->stream, u);
-  }
+  if (c->diff_on && Ud)
+    launch_update_d<kDiagBlocks>(c, u);
+  else if (u.diag)
+    launch_update_d<kDiagFull>(c, u);
+  else
+    launch_update_d<kDiagNone>(c, u);
   HIPCHK(c, hipGetLastError());
   return 0;
 }
 
 // ------------------------------------------------------------- diffusion
-// The setup kernel over every vertex: the small class with its matrices in
-// dynamic LDS in one launch; the large class with them in the workspace,
-// kDiffWsBlocks vertices per launch.
-void launch_diff_setup(subfv_ctx *c, DiffArgs a) {
-  a.set_fm = c->diff_fm;
-  a.set_em = c->diff_em;
-  const long V = c->dm.V;
-  if (!c->diff_large) {
-    a.v0 = 0;
-    hipLaunchKernelGGL((k_diff_setup<kDiffMaxSub, false>), dim3((unsigned)V), dim3(64),
-                       diff_setup_lds_bytes(a.set_fm, a.set_em), c->stream, a);
-    return;
-  }
-  a.ws = c->dws;
-  a.ws_stride = diff_setup_ws_stride(a.set_fm, a.set_em);
-  for (long v0 = 0; v0 < V; v0 += kDiffWsBlocks) {
-    a.v0 = (int)v0;
-    hipLaunchKernelGGL((k_diff_setup<kDiffMaxSubL, true>), dim3((unsigned)std::min<long>(kDiffWsBlocks, V - v0)),
-                       dim3(64), 0, c->stream, a);
-  }
+// the viscous kernels' arguments that depend on the mesh and the parameters
+DiffArgs diff_args(subfv_ctx *c) {
+  DiffArgs a{};
+  a.m = c->dm;
+  a.p = c->dparams;
+  a.doff = c->doff;
+  a.pre = c->pre;
+  a.PD = c->PD;
+  a.rdiff = c->rdiff;
+  a.dblk = c->dblk;
+  a.U = c->U[c->cur];
+  a.scode = c->dscode;
+  a.sivol = c->dsivol;
+  a.fpos = c->dfpos;
+  a.nim = c->diff_nim;
+  a.nfm = c->diff_nfm;
+  a.nsm = c->diff_nsm;
+  a.lmat = c->diff_lmat;
+  a.parts = 3;
+  return a;
 }
 
-// Once per mesh and parameter set: offsets of the packed per-vertex blocks,
-// buffers, and the setup kernel (nodal systems, inverses, products).
+// Once per mesh: the kernels' tables, each vertex's place in the packed
+// inverses, and the size class; once per mesh and parameter set with a
+// constant viscosity: the inverses of the nodal systems.
 int ensure_diffusion(subfv_ctx *c) {
   if (c->diff_ready) return 0;
   const subfv::HostMesh &h = *c->hmp;
   if (h.periodic) return fail(c, SUBFV_E_INVALID, "viscous terms are not available on periodic meshes");
-  std::vector<long> off(h.nv + 1, 0);
-  int mf = 1, me = 1;
-  for (int v = 0; v < h.nv; v++) {
-    const int nf = h.sf_off[v + 1] - h.sf_off[v], ns = h.v_seoff[v + 1] - h.v_seoff[v];
-    if (nf > kDiffMaxSubL || ns > kDiffMaxSubL)
-      return fail(c, SUBFV_E_INVALID, "viscous terms: vertex " + std::to_string(v + 1) + " has more than " +
-                                          std::to_string(kDiffMaxSubL) + " sub-faces or sub-elements");
-    off[v + 1] = off[v] + diff_block_size(nf, ns);
-    mf = std::max(mf, nf);
-    me = std::max(me, ns);
-  }
-  c->diff_fm = 3 * mf;
-  c->diff_em = 3 * me;
-  c->diff_large = mf > kDiffMaxSub || me > kDiffMaxSub;
-  const size_t lds = diff_setup_lds_bytes(c->diff_fm, c->diff_em);
-  if (!c->diff_large && lds > (64u << 10))
-    HIPCHK(c, hipFuncSetAttribute((const void *)k_diff_setup<kDiffMaxSub, false>,
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   int r;
   // the buffers' sizes depend on the mesh only: allocated once per mesh and
   // kept when the viscous parameters change (a new mesh resets them)
   if (!c->doff) {
-    size_t free_b = 0, total_b = 0;
-    HIPCHK(c, hipMemGetInfo(&free_b, &total_b));
-    const size_t need = sizeof(double) * ((size_t)off[h.nv] + (size_t)kDiffSlot * h.nse + 29ull * h.ne);
-    if (need + ((size_t)1 << 30) > free_b)
-      return fail(c, SUBFV_E_DEVICE, "viscous terms: " + std::to_string(need >> 20) + " MiB needed, " +
-                                         std::to_string(free_b >> 20) + " MiB free");
+    int mf = 1, me = 1;
+    for (int v = 0; v < h.nv; v++) {
+      const int nf = h.sf_off[v + 1] - h.sf_off[v], ns = h.v_seoff[v + 1] - h.v_seoff[v];
+      if (nf > kDiffMaxSub || ns > kDiffMaxSub)
+        return fail(c, SUBFV_E_INVALID, "viscous terms: vertex " + std::to_string(v + 1) + " has more than " +
+                                            std::to_string(kDiffMaxSub) + " sub-faces or sub-elements");
+      mf = std::max(mf, nf);
+      me = std::max(me, ns);
+    }
+    const size_t fixed = sizeof(double) * ((size_t)(kDiffSlot + 2) * h.nse + (29ull + kDiffBlk) * h.ne + 2ull * h.nv) + h.nsf;
+    auto room = [&](size_t need) -> int {
+      size_t free_b = 0, total_b = 0;
+      HIPCHK(c, hipMemGetInfo(&free_b, &total_b));
+      if (need + ((size_t)1 << 30) > free_b)
+        return fail(c, SUBFV_E_DEVICE, "viscous terms: " + std::to_string(need >> 20) + " MiB needed, " +
+                                           std::to_string(free_b >> 20) + " MiB free");
+      return 0;
+    };
+    if ((r = room(fixed))) return r;
+    int *vstat = nullptr;
+    if ((r = dalloc(c, &vstat, (size_t)h.nv))) return r;
+    if ((r = dalloc(c, &c->dfpos, (size_t)h.nsf))) return r;
+    if ((r = dalloc(c, &c->dscode, (size_t)h.nse))) return r;
+    if ((r = dalloc(c, &c->dsivol, (size_t)h.nse))) return r;
+    launch_diff_tables(c->dm, vstat, c->dfpos, c->dscode, c->dsivol, c->stream);
+    HIPCHK(c, hipGetLastError());
+    std::vector<int> st(h.nv);
+    HIPCHK(c, hipMemcpyAsync(st.data(), vstat, sizeof(int) * h.nv, hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    int nim = 1;
+    for (int v = 0; v < h.nv; v++) nim = std::max(nim, st[v] & 0xFF);
+    // 32 lanes per vertex hold a row of its inverse each (3 stored faces x 3
+    // <= 30 rows) while it is formed, 64 lanes up to 63 rows
+    c->diff_cls = nim <= 10 && me <= 16 ? kDiffHalf : (nim <= 21 ? kDiffWave : kDiffLarge);
+    c->diff_nim = nim;
+    c->diff_nfm = mf;
+    c->diff_nsm = me;
+    // doubles of each vertex's inverses: 3x3 blocks and heat entries on and
+    // below the diagonal, or all where the vertex is tagged; the large class
+    // reserves all (its inverses for cell viscosities are stored too)
+    std::vector<uint64_t> off(h.nv);
+    uint64_t at = 0;
+    int lmat = 1;
+    for (int v = 0; v < h.nv; v++) {
+      const uint64_t ni = st[v] & 0xFF, tag = st[v] >> 8;
+      const uint64_t nb = tag || c->diff_cls == kDiffLarge ? ni * ni : ni * (ni + 1) / 2;
+      off[v] = at | ni << 48 | tag << 56;
+      lmat = std::max(lmat, (int)(10 * nb));
+      at += 10 * nb;
+    }
+    c->diff_lmat = lmat;
+    if ((r = room(fixed + sizeof(double) * at))) return r;
     if ((r = upload(c, &c->doff, off))) return r;
-    if ((r = dalloc(c, &c->pre, (size_t)off[h.nv]))) return r;
-    c->pre_n = off[h.nv];
+    if ((r = dalloc(c, &c->pre, (size_t)at))) return r;
+    c->pre_n = (long)at;
     if ((r = dalloc(c, &c->PD, (size_t)kDiffSlot * h.nse))) return r;
     if ((r = dalloc(c, &c->rdiff, 4ull * h.ne))) return r;
-    // each slot's sub-element sub-faces as vertex-local indices, one byte
-    // each in list order (0xFF ends the list), and its volume: the apply
-    // reads them at the slot's index instead of through the cell-major lists
-    std::vector<uint32_t> ssf(h.nse, 0xFFFFFFFFu);
-    for (int v = 0; v < h.nv; v++)
-      for (int q = h.v_seoff[v]; q < h.v_seoff[v + 1]; q++) {
-        const int se = h.v_se[q], pb = h.se_sfoff[se], pe = h.se_sfoff[se + 1];
-        if (pe - pb > kSlotSrc)
-          return fail(c, SUBFV_E_INVALID, "viscous terms: a sub-element has more than " +
-                                              std::to_string(kSlotSrc) + " sub-faces");
-        for (int pp = pb; pp < pe; pp++) {
-          const uint32_t loc = (uint32_t)(h.se_sf[pp] - h.sf_off[v]);
-          ssf[q] &= ~(0xFFu << (8 * (pp - pb)));
-          ssf[q] |= loc << (8 * (pp - pb));
-        }
-      }
-    if ((r = upload(c, &c->dssf, ssf))) return r;
-    if (c->diff_large &&
-        (r = dalloc(c, &c->dws, (size_t)kDiffWsBlocks * diff_setup_ws_stride(c->diff_fm, c->diff_em))))
-      return r;
-    if ((r = dalloc(c, &c->dsvol, (size_t)h.nse))) return r;
-    hipLaunchKernelGGL(k_slot_vol, dim3(nblk(h.nse, 256)), dim3(256), 0, c->stream, (long)h.nse,
-                       (const int *)c->dm.v_seid, (const double *)c->dm.se_vol, c->dsvol);
+    if ((r = dalloc(c, &c->dblk, (size_t)kDiffBlk * h.ne))) return r;
   }
   if (c->dparams.suth && !c->mu_cell) {
     if ((r = dalloc(c, &c->mu_cell, (size_t)h.ne))) return r;
@@ -758,18 +776,8 @@ int ensure_diffusion(subfv_ctx *c) {
   if (!c->diag && (r = dalloc(c, &c->diag, 25ull * h.ne))) return r;
   HIPCHK(c, hipMemsetAsync(c->diag, 0, sizeof(double) * 25 * h.ne, c->stream));
   HIPCHK(c, hipMemsetAsync(c->rdiff, 0, sizeof(double) * 4 * h.ne, c->stream));
-  DiffArgs a{};
-  a.m = c->dm;
-  a.p = c->dparams;
-  a.doff = c->doff;
-  a.pre = c->pre;
-  a.U = nullptr;
-  a.PD = c->PD;
-  a.rdiff = c->rdiff;
-  a.diag = c->diag;
-  // with Sutherland's law the blocks depend on the state: formed per residual
-  if (!c->dparams.suth) launch_diff_setup(c, a);
-  HIPCHK(c, hipGetLastError());
+  // with Sutherland's law the inverses depend on the state: formed per residual
+  if (!c->dparams.suth) HIPCHK(c, launch_diff_setup(c->diff_cls, diff_args(c), c->stream));
   c->diff_ready = true;
   return 0;
 }
@@ -798,33 +806,22 @@ __global__ __launch_bounds__(kCellThreads) void k_mu_min(const double *blk, int 
 
 // rdiff and diag of the state U (build_momentum_diff_mat_into_global_mat_diag
 // and build_diff_mat_into_global_mat_diag).  mu_cell / mu_min: given cell viscosities
-// and their mu0corr (device), for which the nodal systems are formed anew
-// (the constant-viscosity blocks are then invalidated); parts: 1 momentum,
-// 2 heat, 3 both.
+// and their mu0corr (device), for which the nodal systems are formed anew;
+// parts: 1 momentum, 2 heat, 3 both.
 int launch_diffusion(subfv_ctx *c, const double *U, const double *mu_cell = nullptr,
                      const double *mu_min = nullptr, int parts = 3) {
   int r = ensure_diffusion(c);
   if (r) return r;
-  DiffArgs a{};
+  DiffArgs a = diff_args(c);
   a.parts = parts;
-  a.m = c->dm;
-  a.p = c->dparams;
-  a.doff = c->doff;
-  a.pre = c->pre;
   a.U = U;
-  a.PD = c->PD;
-  a.rdiff = c->rdiff;
-  a.diag = c->diag;
-  a.slot_ssf = c->dssf;
-  a.slot_vol = c->dsvol;
   Prof pf(c, "diffusion");
   if (mu_cell) {
     a.mu_cell = mu_cell;
     a.mu_min = mu_min;
-    launch_diff_setup(c, a);
-    if (!c->dparams.suth) c->diff_ready = false;  // the cached constant-viscosity blocks are overwritten
+    a.pivot = 1;  // any mu0corr: the systems need not be positive definite
+    if (!c->dparams.suth) c->diff_ready = false;  // the constant-viscosity blocks and inverses are overwritten
   } else if (c->dparams.suth) {
-    Prof ps(c, "diff_setup");
     const unsigned nb = nblk(c->dm.C, kCellThreads);
     hipLaunchKernelGGL(k_compute_mu, dim3(nb), dim3(kCellThreads), 0, c->stream, (long)c->dm.C, U, c->dparams.cv,
                        c->dparams.suth_mu0, c->dparams.suth_T0, c->mu_cell, c->mu_blk);
@@ -832,27 +829,18 @@ int launch_diffusion(subfv_ctx *c, const double *U, const double *mu_cell = null
                        c->mu_blk + nb);
     a.mu_cell = c->mu_cell;
     a.mu_min = c->mu_blk + nb;
-    launch_diff_setup(c, a);
   }
-  const int waves = c->diff_large ? 1 : kDiffWaves;
-  a.vblocks = (int)nblk(c->dm.V, waves);
-  a.vper_xcd = (a.vblocks + 7) / 8;
-  a.cblocks = (int)nblk(c->dm.C, kDgCells);
-  a.cper_xcd = (a.cblocks + 7) / 8;
   {
     Prof pa(c, "diff_apply");
-    if (c->diff_large)
-      hipLaunchKernelGGL((k_diff_apply<kDiffMaxSubL, kDiffMaxSubL, kDiffStage, 1, 7>), dim3(8 * a.vper_xcd),
-                         dim3(64), 0, c->stream, a);
-    else if (c->diff_em <= 3 * kDiffMaxSubC)
-      hipLaunchKernelGGL((k_diff_apply<kDiffMaxSub, kDiffMaxSubC, kDiffStageC, kDiffWaves, 8>),
-                         dim3(8 * a.vper_xcd), dim3(64 * kDiffWaves), 0, c->stream, a);
-    else
-      hipLaunchKernelGGL((k_diff_apply<kDiffMaxSub, kDiffMaxSub, kDiffStage, kDiffWaves, 7>), dim3(8 * a.vper_xcd),
-                         dim3(64 * kDiffWaves), 0, c->stream, a);
+    HIPCHK(c, launch_diff_terms(c->diff_cls, a, c->stream));
   }
-  hipLaunchKernelGGL(k_diff_gather, dim3(8 * a.cper_xcd), dim3(256), 0, c->stream, a);
-  HIPCHK(c, hipGetLastError());
+  HIPCHK(c, launch_diff_gather(a, c->stream));
+  return 0;
+}
+
+// the diag array of the residual state U, for callers that read it
+int expand_diag(subfv_ctx *c, const double *U) {
+  HIPCHK(c, launch_diff_expand(c->dm.C, U, c->dblk, c->dparams.cv, c->diag, c->stream));
   return 0;
 }
 
@@ -1408,6 +1396,7 @@ int subfv_compute_rhs_ns(subfv_ctx *c) {
     // the diffusion block (ns_main.F90:170-175): rhs += viscous terms, diag = their block
     r = launch_diffusion(c, c->U[c->cur]);
     if (r) return r;
+    if ((r = expand_diag(c, c->U[c->cur]))) return r;
     hipLaunchKernelGGL(k_add_rdiff, dim3(nblk(c->dm.C, 256)), dim3(256), 0, c->stream, (long)c->dm.C, c->rhs,
                        (const double *)c->rdiff);
     HIPCHK(c, hipGetLastError());
@@ -1694,6 +1683,7 @@ int subfv_add_diffusion(subfv_ctx *c, const double *sol, const double *mu_arr, d
   HIPCHK(c, hipMemcpyAsync(c->mu_cell, mu_arr, C * sizeof(double), hipMemcpyHostToDevice, s));
   HIPCHK(c, hipMemcpyAsync(c->mu_blk + nb, &mu0corr, sizeof(double), hipMemcpyHostToDevice, s));
   if ((r = launch_diffusion(c, c->U[c->cur], c->mu_cell, c->mu_blk + nb, parts))) return r;
+  if ((r = expand_diag(c, c->U[c->cur]))) return r;
   Scratch sc;
   double *drhs, *ddiag;
   HIPCHK(c, sc.get(&drhs, 5 * C));
@@ -1715,30 +1705,38 @@ int subfv_run(subfv_ctx *c, int32_t n_steps, int32_t time_scheme, double *t, dou
     return fail(c, SUBFV_E_INVALID, "SSP-RK3 needs local_time_step = .false.");
   int r;
   const int fl = c->cfg.second_order ? 1 : 0;
+  // no stage writes the state its residual was taken at: the update and its
+  // correction read that state again for the viscous diagonal
+  const double *last = nullptr;
   for (int it = 0; it < n_steps; it++) {
     int a = c->cur, b = (a + 1) % 3, q = (a + 2) % 3;
     if (time_scheme == 0) {
       if ((r = residual(c, c->U[a], 0))) return r;
       if (c->cfg.second_order) {
         // ns_main.F90:88-95: half step into U*, residual at U*, full step from U^n
-        if ((r = launch_update(c, c->U[a], nullptr, c->U[b], 2.0, 1.0, 0.0, 1.0, fl, 0, true))) return r;
+        if ((r = launch_update(c, c->U[a], nullptr, c->U[b], 2.0, 1.0, 0.0, 1.0, fl, 0, c->U[a]))) return r;
         if ((r = residual(c, c->U[b], 0))) return r;
-        if ((r = launch_update(c, c->U[a], nullptr, c->U[b], 1.0, 1.0, 0.0, 1.0, fl, 1, true))) return r;
+        if ((r = launch_update(c, c->U[a], nullptr, c->U[q], 1.0, 1.0, 0.0, 1.0, fl, 1, c->U[b]))) return r;
+        last = c->U[b];
+        c->cur = q;
       } else {
-        if ((r = launch_update(c, c->U[a], nullptr, c->U[b], 1.0, 1.0, 0.0, 1.0, 0, 1, true))) return r;
+        if ((r = launch_update(c, c->U[a], nullptr, c->U[b], 1.0, 1.0, 0.0, 1.0, 0, 1, c->U[a]))) return r;
+        last = c->U[a];
+        c->cur = b;
       }
-      c->cur = b;
     } else {
       // SSP-RK3: U1 = L(Un) -> b; U2 = 3/4 Un + 1/4 L(U1) -> q; Un+1 = 1/3 Un + 2/3 L(U2) -> b
       if ((r = residual(c, c->U[a], 0))) return r;
-      if ((r = launch_update(c, c->U[a], nullptr, c->U[b], 1.0, 1.0, 0.0, 1.0, fl, 0, true))) return r;
+      if ((r = launch_update(c, c->U[a], nullptr, c->U[b], 1.0, 1.0, 0.0, 1.0, fl, 0, c->U[a]))) return r;
       if ((r = residual(c, c->U[b], 1))) return r;
-      if ((r = launch_update(c, c->U[b], c->U[a], c->U[q], 1.0, 1.0, 0.75, 0.25, fl, 0, true))) return r;
+      if ((r = launch_update(c, c->U[b], c->U[a], c->U[q], 1.0, 1.0, 0.75, 0.25, fl, 0, c->U[b]))) return r;
       if ((r = residual(c, c->U[q], 1))) return r;
-      if ((r = launch_update(c, c->U[q], c->U[a], c->U[b], 1.0, 1.0, 1.0 / 3.0, 2.0 / 3.0, fl, 2, true))) return r;
+      if ((r = launch_update(c, c->U[q], c->U[a], c->U[b], 1.0, 1.0, 1.0 / 3.0, 2.0 / 3.0, fl, 2, c->U[q]))) return r;
+      last = c->U[q];
       c->cur = b;
     }
   }
+  if (last && c->diff_on && (r = expand_diag(c, last))) return r;
   StepState hs;
   r = sync_state_scalars(c, &hs);
   if (r) return r;

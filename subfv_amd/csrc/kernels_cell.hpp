@@ -4,6 +4,7 @@
 // second-order reconstruction.
 #pragma once
 #include "device_mesh.hpp"
+#include "kernels_diff.hpp"
 #include "kernels_flux.hpp"
 #include "physics.hpp"
 
@@ -177,7 +178,9 @@ struct UpdateArgs {
   const double *U0;   // combination partner (w0 != 0) or null
   double *Uout;       // [C][5]
   const double *rhs, *rhs2, *sl;
-  const double *diag; // [C][25] column-major 5x5 blocks, or null (c*I diagonal)
+  const double *diag; // [C][25] column-major 5x5 blocks (kDiagFull)
+  const double *Ud, *dblk;  // the residual's state and the cells' viscous blocks (kDiagBlocks)
+  double cv;
   const double *rdiff;// [C][4] viscous rhs of components 2..5 (added after flux limiting), or null
   double *blk;
   StepState *st;
@@ -186,10 +189,14 @@ struct UpdateArgs {
   int advance_t;      // closes a step: 1 -> t += dt_adv (reference), 2 -> t += dt
 };
 
+// the diagonal of a stage update: c*I; the given diag array; or c*I plus the
+// viscous block formed from the cell's mesh-constant (or just gathered) sums
+enum { kDiagNone = 0, kDiagFull = 1, kDiagBlocks = 2 };
+
 // flux_limiting (ns_euler_recon_module.F90:586-593) + the per-cell part of
 // add_timedisc_and_solve (ns_euler_module.F90:565-580).  Returns the cell's
 // omega; u and delta receive the state and the increment.
-template <bool DIAG>
+template <int DIAG>
 SFV_DEV double stage_cell(const UpdateArgs &a, const double *U, long c, double *u, double *delta) {
   const long C = a.m.C;
   const StepState *st = a.st;
@@ -217,7 +224,10 @@ SFV_DEV double stage_cell(const UpdateArgs &a, const double *U, long c, double *
   double nw[5];
   if (DIAG) {
     double D[25];
-    for (int q = 0; q < 25; q++) D[q] = a.diag[25 * c + q];
+    if (DIAG == kDiagBlocks)
+      diff_block(a.Ud + 5 * c, a.dblk + (long)kDiffBlk * c, a.cv, D);
+    else
+      for (int q = 0; q < 25; q++) D[q] = a.diag[25 * c + q];
     for (int q = 0; q < 5; q++) D[q + 5 * q] = D[q + 5 * q] + cc;
     double b[5];
     for (int k = 0; k < 5; k++) b[k] = r[k] + cc * u[k];
@@ -243,7 +253,7 @@ SFV_DEV void store_stage(const UpdateArgs &a, double *Uout, long c, const double
   }
 }
 
-template <bool DIAG>
+template <int DIAG>
 SFV_DEV void update_block(const UpdateArgs &a, const double *U, double *Uout, long bidx) {
   long c = bidx * kCellThreads + threadIdx.x;
   StepState *st = a.st;
@@ -261,14 +271,14 @@ SFV_DEV void update_block(const UpdateArgs &a, const double *U, double *Uout, lo
   block_min_store(om_c, a.blk, (int)bidx);
 }
 
-template <bool DIAG>
+template <int DIAG>
 __global__ __launch_bounds__(kCellThreads) void k_update(UpdateArgs a) {
   update_block<DIAG>(a, a.U, a.Uout, blockIdx.x);
 }
 
 // Correction when the global omega came out below one: redo the cell with
 // sol = sol + a2*omega*delta (ns_euler_module.F90:608).
-template <bool DIAG>
+template <int DIAG>
 SFV_DEV void update_fixup_block(const UpdateArgs &a, const double *U, double *Uout, long bidx) {
   long c = bidx * kCellThreads + threadIdx.x;
   const StepState *st = a.st;
@@ -279,7 +289,7 @@ SFV_DEV void update_fixup_block(const UpdateArgs &a, const double *U, double *Uo
   store_stage(a, Uout, c, u, d, st->omega);
 }
 
-template <bool DIAG>
+template <int DIAG>
 __global__ __launch_bounds__(kCellThreads) void k_update_fixup(UpdateArgs a) {
   update_fixup_block<DIAG>(a, a.U, a.Uout, blockIdx.x);
 }

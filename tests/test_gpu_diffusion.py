@@ -1,13 +1,13 @@
-"""Viscous terms on the device (kernels_diff.hpp) against the oracle
-(om_diffusion.c).  The device forms the nodal products once per mesh and
-adds each cell's terms as one sum per vertex, where the reference adds them
-one by one; results agree to round-off, not bit for bit: the residual within
+"""Viscous terms on the device (diffusion.hip) against the oracle
+(om_diffusion.c).  The device keeps the inverses of the nodal systems and
+adds each cell's terms as one sum per vertex, where the reference multiplies
+dense matrices and adds the terms one by one; results agree to round-off, not bit for bit: the residual within
 1e-12 of the viscous terms' scale (measured: 2e-14 on tri 8^2, 4e-17 for the
 point-implicit diagonal) and the state after 100 viscous steps within 1e-12
 relative (measured: 1e-15 on tri, quad, 3-D hex and a 10-sub-element fan).
 Tetrahedral meshes (36 sub-faces and 24 sub-elements at an interior vertex)
-take the large-class kernels: setup matrices in a global workspace, one
-vertex per apply workgroup."""
+take the large-class kernels: inverses formed by a workgroup per vertex and
+read from HBM."""
 import numpy as np
 import pytest
 
@@ -150,6 +150,42 @@ def test_viscous_100_steps_within_1e12(solver, name, ts):
     assert st == 0
     rel = np.abs(got - ref).max() / np.abs(ref).max()
     assert rel <= 1e-12, rel
+
+
+# (k, layers): the axis vertex between two layers has 2k sub-elements and 3k
+# faces, all with unknowns of their own; with one layer k sub-elements, k such
+# faces and k derived wall faces.  Edges of the size classes: 10 | 11 (32 or 64
+# lanes per vertex), 21 | 22 and 24 (inverses in HBM), 37 | 39 (larger tiles),
+# 63 (the most a byte code holds is 64).
+@pytest.mark.parametrize("law", ["constant", "sutherland"])
+@pytest.mark.parametrize("k,layers", [(3, 1), (10, 1), (11, 1), (7, 2), (22, 1), (8, 2), (13, 2), (21, 2)])
+def test_vertex_size_classes_match_oracle(solver, k, layers, law):
+    """rhs and diag of one residual within 1e-12 of the viscous terms' scale,
+    as for the meshes above."""
+    print(f"[gpu] viscous class fan k={k} layers={layers} {law}", flush=True)
+    mesh = fan_prism_mesh(k, layers)
+    solver.build_mesh(mesh)
+    om = O.OracleMesh(mesh)
+    suth = law == "sutherland"
+    sol = warm_state(om.elem_coord) if suth else smooth_state(om.elem_coord)
+    kw = dict(boundary_2d=False, second_order=False)
+    solver.set_config(make_config("multi_point", **kw))
+    solver.set_diffusion(True, mu=2e-3)
+    solver.set_sutherland(suth)
+    try:
+        solver.put_sol(sol)
+        solver.compute_rhs_ns()
+        rhs, diag = solver.get("rhs"), solver.get("diag")
+    finally:
+        solver.set_sutherland(False)
+        solver.set_diffusion(False)
+    ocfg = O.make_config("multi_point", diffusion=True, mu=2e-3, sutherland=suth, **kw)
+    r0, _ = om.compute_euler_flux(ocfg, sol)
+    rd, dd = om.add_diffusion(ocfg, sol)
+    scale = np.abs(rd).max(axis=0) + 1e-300
+    assert np.all(np.abs(rhs - (r0 + rd)) <= 1e-12 * scale[None, :] + 1e-14 * np.abs(r0 + rd)), \
+        np.abs(rhs - r0 - rd).max(axis=0) / scale
+    assert np.abs(diag - dd).max() <= 1e-12 * np.abs(dd).max()
 
 
 def test_vertices_beyond_the_limit_are_rejected(solver):
