@@ -924,20 +924,54 @@ int mesh_i32(const subfv::HostMesh &h, const char *name, int32_t *out, int64_t c
   return (int64_t)v.size();
 }
 
+// [ncomp][n] on the device to the reference's [n][ncomp] and back; one lane per
+// interleaved value
+__global__ __launch_bounds__(256) void k_interleave(int ncomp, long n, const double *soa, double *aos) {
+  const long q = (long)blockIdx.x * 256 + threadIdx.x;
+  if (q < ncomp * n) aos[q] = soa[(q % ncomp) * n + q / ncomp];
+}
+__global__ __launch_bounds__(256) void k_deinterleave(int ncomp, long n, const double *aos, double *soa) {
+  const long q = (long)blockIdx.x * 256 + threadIdx.x;
+  if (q < ncomp * n) soa[(q % ncomp) * n + q / ncomp] = aos[q];
+}
+
+// Device arrays to and from host memory in the reference's layout: copied
+// straight between the device and the caller's array (a 2.1M-cell state: 8 ms
+// out into fresh pages and 3 ms in, where a vector in between and a host loop
+// took 55 ms), component arrays interleaved on the device first.  c->P, the node
+// sweep's partials, is free outside a residual and holds them where it is large
+// enough (8 values per sub-element: 5 per cell and 3 per vertex always fit, 3
+// per sub-face on all but meshes of a few cells).
+bool fits_partials(const subfv_ctx *c, int ncomp, long n) { return ncomp * n <= kSlotStride * c->dm.SE; }
+
 int dev_to_host_soa(subfv_ctx *c, const double *d, int ncomp, long n, double *out) {
-  std::vector<double> tmp((size_t)ncomp * n);
-  HIPCHK(c, hipMemcpyAsync(tmp.data(), d, tmp.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+  if (ncomp > 1 && !fits_partials(c, ncomp, n)) {
+    std::vector<double> tmp((size_t)ncomp * n);
+    HIPCHK(c, hipMemcpyAsync(tmp.data(), d, tmp.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    for (long i = 0; i < n; i++)
+      for (int k = 0; k < ncomp; k++) out[(size_t)i * ncomp + k] = tmp[(size_t)k * n + i];
+    return 0;
+  }
+  if (ncomp > 1) {
+    hipLaunchKernelGGL(k_interleave, dim3(nblk(ncomp * n, 256)), dim3(256), 0, c->stream, ncomp, n, d, c->P);
+    HIPCHK(c, hipGetLastError());
+    d = c->P;
+  }
+  HIPCHK(c, hipMemcpyAsync(out, d, sizeof(double) * ncomp * n, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
-  for (long i = 0; i < n; i++)
-    for (int k = 0; k < ncomp; k++) out[(size_t)i * ncomp + k] = tmp[(size_t)k * n + i];
   return 0;
 }
 
 int host_to_dev_soa(subfv_ctx *c, const double *in, int ncomp, long n, double *d) {
-  std::vector<double> tmp((size_t)ncomp * n);
-  for (long i = 0; i < n; i++)
-    for (int k = 0; k < ncomp; k++) tmp[(size_t)k * n + i] = in[(size_t)i * ncomp + k];
-  HIPCHK(c, hipMemcpyAsync(d, tmp.data(), tmp.size() * sizeof(double), hipMemcpyHostToDevice, c->stream));
+  if (ncomp > 1 && !fits_partials(c, ncomp, n)) return fail(c, SUBFV_E_INVALID, "more values than the mesh holds");
+  double *to = ncomp > 1 ? c->P : d;
+  HIPCHK(c, hipMemcpyAsync(to, in, sizeof(double) * ncomp * n, hipMemcpyHostToDevice, c->stream));
+  if (ncomp > 1) {
+    hipLaunchKernelGGL(k_deinterleave, dim3(nblk(ncomp * n, 256)), dim3(256), 0, c->stream, ncomp, n,
+                       (const double *)to, d);
+    HIPCHK(c, hipGetLastError());
+  }
   HIPCHK(c, hipStreamSynchronize(c->stream));
   return 0;
 }
