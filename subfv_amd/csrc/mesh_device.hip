@@ -168,6 +168,182 @@ __global__ void k_bfs_assign(int n, const int *sorted, int iloc, int *otn, int *
   }
 }
 
+// Whole levels by one workgroup, without host reads or sorts: while the
+// frontier has at most kBfsCap vertices.  Eight lanes take a frontier vertex, an
+// element each.  (1) an unvisited vertex keeps the smallest key (place of the
+// frontier vertex, its element, the corner) that meets it, the reference's scan
+// order; (2) each frontier vertex counts the vertices whose kept key is its own;
+// (3) the counts' prefix sums number them, (4) in the order of its scan.  With
+// nothing reached the lowest unvisited vertex starts the next component.
+// pos: iloc, istart, iend, first vertex that may be unvisited.
+// A level is a few hundred vertices: as launches with a sort and a host read it
+// took about 110 us (tri 200^2, 238 levels), here 30 us, the scattered accesses
+// of one CU (each step reads every corner's mark; keeping the corners in
+// registers between the steps did not help, 39 us with the half as many
+// threads that they leave room for).  Larger frontiers fill more than one CU
+// and keep the level-wise kernels above.
+constexpr int kBfsCap = 2048;
+constexpr int kBfsThreads = 1024;
+__global__ __launch_bounds__(kBfsThreads) void k_bfs_levels(int nv, const int *v_eoff, const int *v_elem,
+                                                            const int *e_voff, const int *e_vert, int *otn, int *nto,
+                                                            unsigned long long *prio, int *pos) {
+  __shared__ int base[kBfsCap];
+  __shared__ int wsum[kBfsThreads / 64];
+  __shared__ int s_first;
+  constexpr int kPer = kBfsThreads / 8;  // frontier vertices per round
+  const int tid = threadIdx.x, sub = tid & 7, lane = tid & 63, wv = tid >> 6;
+  // written by atomics or other waves: read past the L1 cache
+  auto unvisited = [&](int w) { return __hip_atomic_load(&otn[w], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < 0; };
+  auto kept = [&](int w) { return __hip_atomic_load(&prio[w], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+  // the atomics and stores of the step have reached L2
+  auto sync_level = [] {
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+  };
+  auto key = [](int i, int k, int r) { return (unsigned long long)i << 32 | (unsigned)(k << 3 | r); };
+  // the corners of an element, loaded together (-1 past the last)
+  auto corners = [&](int q, int *w) {
+    const int el = v_elem[q], rb = e_voff[el], n = e_voff[el + 1] - rb;
+#pragma unroll
+    for (int r = 0; r < 8; r++) w[r] = r < n ? e_vert[rb + r] : -1;
+  };
+  auto claim = [&](const int *w, int i, int k) {
+    bool free[8];
+#pragma unroll
+    for (int r = 0; r < 8; r++) free[r] = w[r] >= 0 && unvisited(w[r]);
+#pragma unroll
+    for (int r = 0; r < 8; r++)
+      if (free[r]) atomicMin(&prio[w[r]], key(i, k, r));
+  };
+  // which of the corners kept the key of this place
+  auto wins = [&](const int *w, int i, int k) {
+    unsigned long long x[8];
+    unsigned won = 0;
+#pragma unroll
+    for (int r = 0; r < 8; r++) x[r] = w[r] >= 0 ? kept(w[r]) : ~0ull;
+#pragma unroll
+    for (int r = 0; r < 8; r++)
+      if (x[r] == key(i, k, r)) won |= 1u << r;
+    return won;
+  };
+  // numbers the won corners from `at` in lane order; returns how many the eight lanes won
+  auto assign = [&](const int *w, unsigned won, int at) {
+    const int c = __popc(won);
+    int x = c;
+    for (int o = 1; o < 8; o <<= 1) {
+      const int y = __shfl_up(x, o, 8);
+      if (sub >= o) x += y;
+    }
+    int k = at + x - c;
+#pragma unroll
+    for (int r = 0; r < 8; r++)
+      if (won >> r & 1) {
+        __hip_atomic_store(&otn[w[r]], k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        // keys count from each level's frontier: none may outlive its level
+        __hip_atomic_store(&prio[w[r]], ~0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        nto[k++] = w[r];
+      }
+    return __shfl(x, 7, 8);
+  };
+  int iloc = pos[0], istart = pos[1], iend = pos[2], cursor = pos[3];
+  while (iloc < nv) {
+    const int nfront = iend - istart + 1;
+    if (nfront > kBfsCap) break;
+    for (int i = tid >> 3; i < nfront; i += kPer) {
+      const int v = nto[istart + i], b = v_eoff[v], e = v_eoff[v + 1];
+      for (int q = b + sub; q < e; q += 8) {
+        int w[8];
+        corners(q, w);
+        claim(w, i, q - b);
+      }
+    }
+    sync_level();
+    for (int i = tid >> 3; i < nfront; i += kPer) {
+      const int v = nto[istart + i], b = v_eoff[v], e = v_eoff[v + 1];
+      int c = 0;
+      for (int q = b + sub; q < e; q += 8) {
+        int w[8];
+        corners(q, w);
+        c += __popc(wins(w, i, q - b));
+      }
+      for (int o = 1; o < 8; o <<= 1) c += __shfl_xor(c, o);
+      if (sub == 0) base[i] = c;
+    }
+    __syncthreads();
+    int found = 0;
+    {  // exclusive prefix sums of base, kEach consecutive entries per thread
+      constexpr int kEach = kBfsCap / kBfsThreads;
+      const int i0 = kEach * tid;
+      int a[kEach], t = 0;
+#pragma unroll
+      for (int k = 0; k < kEach; k++) {
+        a[k] = i0 + k < nfront ? base[i0 + k] : 0;
+        t += a[k];
+      }
+      int x = t;
+      for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(x, o);
+        if (lane >= o) x += y;
+      }
+      if (lane == 63) wsum[wv] = x;
+      __syncthreads();
+      int ex = x - t;
+      for (int k = 0; k < kBfsThreads / 64; k++) {
+        if (k < wv) ex += wsum[k];
+        found += wsum[k];
+      }
+#pragma unroll
+      for (int k = 0; k < kEach; k++) {
+        if (i0 + k < nfront) base[i0 + k] = ex;
+        ex += a[k];
+      }
+    }
+    __syncthreads();
+    for (int i = tid >> 3; i < nfront; i += kPer) {
+      const int v = nto[istart + i], b = v_eoff[v], e = v_eoff[v + 1];
+      int at = iloc + base[i];
+      for (int q0 = b; q0 < e; q0 += 8) {  // eight elements at a time, in order
+        const int q = q0 + sub;
+        int w[8];
+#pragma unroll
+        for (int r = 0; r < 8; r++) w[r] = -1;
+        if (q < e) corners(q, w);
+        at += assign(w, wins(w, i, q - b), at);
+      }
+    }
+    if (found == 0) {  // uniform: nothing was assigned in this level
+      for (int q = cursor;; q += kBfsThreads) {  // ends: iloc < nv, so one is unvisited
+        if (tid == 0) s_first = INT_MAX;
+        __syncthreads();
+        if (q + tid < nv && unvisited(q + tid)) atomicMin(&s_first, q + tid);
+        __syncthreads();
+        const int w = s_first;
+        __syncthreads();
+        if (w == INT_MAX && q + kBfsThreads < nv) continue;
+        if (w != INT_MAX) {
+          if (tid == 0) {
+            __hip_atomic_store(&otn[w], iloc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            nto[iloc] = w;
+          }
+          cursor = w + 1;
+        }
+        break;
+      }
+      found = 1;
+    }
+    iloc += found;
+    istart = iend + 1;
+    iend = iloc - 1;
+    sync_level();
+  }
+  if (tid == 0) {
+    pos[0] = iloc;
+    pos[1] = istart;
+    pos[2] = iend;
+    pos[3] = cursor;
+  }
+}
+
 // the lowest index of a negative entry (res starts at INT_MAX)
 __global__ void k_first_negative(int n, const int *a, int *res) {
   GSTRIDE(i, n) if (a[i] < 0) atomicMin(res, (int)i);
@@ -581,6 +757,11 @@ std::string build_device_mesh(HostMesh &m, int nv, const double *coord, int ne, 
   // ---- renumber_vert_mesh: level-synchronous breadth-first search
   Buf<int> otn, nto, prio, list, slist, fcnt, fbase, nlist, res;
   Buf<unsigned> pkey, pkey2;
+  Buf<unsigned long long> prio64;
+  Buf<int> pos;
+  c.chk(prio64.alloc(nv));
+  c.chk(pos.alloc(4));
+  c.chk(hipMemsetAsync(prio64.p, 0xFF, nv * sizeof(unsigned long long), c.s));
   c.chk(otn.alloc(nv));
   c.chk(nto.alloc(nv));
   c.chk(prio.alloc(nv));
@@ -600,8 +781,18 @@ std::string build_device_mesh(HostMesh &m, int nv, const double *coord, int ne, 
     c.chk(hipMemcpyAsync(nto.p, &zero, sizeof(int), hipMemcpyHostToDevice, c.s));
     c.chk(hipStreamSynchronize(c.s));
   }
-  int iloc = 1, istart = 0, iend = 0;
-  while (iloc < nv && !c.err) {
+  int hpos[4] = {1, 0, 0, 0};  // iloc, istart, iend, cursor of k_bfs_levels
+  while (hpos[0] < nv && !c.err) {
+    int &iloc = hpos[0], &istart = hpos[1], &iend = hpos[2];
+    if (iend - istart + 1 <= kBfsCap) {
+      c.chk(hipMemcpyAsync(pos.p, hpos, sizeof(hpos), hipMemcpyHostToDevice, c.s));
+      hipLaunchKernelGGL(k_bfs_levels, dim3(1), dim3(kBfsThreads), 0, c.s, nv, (const int *)v_eoff, (const int *)v_elem,
+                         (const int *)d_evoff, (const int *)d_evert, otn.p, nto.p, prio64.p, pos.p);
+      c.chk(hipGetLastError());
+      c.chk(hipMemcpyAsync(hpos, pos.p, sizeof(hpos), hipMemcpyDeviceToHost, c.s));
+      c.chk(hipStreamSynchronize(c.s));
+      continue;
+    }
     const int nfront = iend - istart + 1;
     int found = 0;
     if (nfront > 0) {
