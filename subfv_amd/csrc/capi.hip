@@ -445,6 +445,10 @@ int upload_mesh(subfv_ctx *c) {
   if ((r = dalloc(c, &d.fnorm, 3L * h.nf))) return r;
   if ((r = dalloc(c, &d.farea, h.nf))) return r;
   if ((r = dalloc(c, &d.sfn, 4L * d.SF))) return r;
+  if ((r = dalloc(c, &d.wsfn, 4L * d.SF))) return r;
+  if ((r = dalloc(c, &d.ws_le, d.SF))) return r;
+  if ((r = dalloc(c, &d.ws_re, d.SF))) return r;
+  if ((r = dalloc(c, &d.ws_id, d.SF))) return r;
   if ((r = dalloc(c, &d.se_vol, h.nse))) return r;
   if ((r = dalloc(c, &d.ccoord, 3L * h.ne))) return r;
   if ((r = dalloc(c, &d.cvol, h.ne))) return r;
@@ -478,6 +482,7 @@ int geometry(subfv_ctx *c) {
   hipLaunchKernelGGL(k_face_centroid, dim3(nblk(d.F, T)), dim3(T), 0, s, d);
   hipLaunchKernelGGL(k_elem_centroid, dim3(nblk(d.C, T)), dim3(T), 0, s, d);
   hipLaunchKernelGGL(k_subface_norm, dim3(nblk(d.SF, T)), dim3(T), 0, s, d);
+  if (d.ngroups) hipLaunchKernelGGL(k_sweep_order, dim3(d.ngroups), dim3(kGrpThreads), 0, s, d);
   hipLaunchKernelGGL(k_face_norm, dim3(nblk(d.F, T)), dim3(T), 0, s, d);
   hipLaunchKernelGGL(k_subelem_volume, dim3(nblk(d.SE, T)), dim3(T), 0, s, d);
   int *bad = c->derr + 1;

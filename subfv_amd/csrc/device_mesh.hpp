@@ -52,6 +52,12 @@ struct DevMesh {
   int *sf_le = nullptr;       // left cell
   int *sf_re = nullptr;       // right code: >=0 cell, -1 wall, <=-2 BC (-code-1)
   double *sfn = nullptr;      // [4][SF]: nx, ny, nz, area
+  // the node sweep's copy: within each vertex group the sub-faces between two
+  // cells come first and the boundary ones last, so that a wavefront holds one
+  // kind (k_sweep_order)
+  double *wsfn = nullptr;     // [4][SF]
+  int *ws_le = nullptr, *ws_re = nullptr;
+  uint16_t *ws_id = nullptr;  // [SF] group-local sub-face and, << 8, group-local vertex
   // sub-elements
   int *se_sfoff = nullptr, *se_sf = nullptr, *se_elem = nullptr;  // cell-major ids
   double *se_vol = nullptr;   // [SE] cell-major

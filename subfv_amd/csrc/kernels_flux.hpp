@@ -11,6 +11,18 @@
 // group run in the first wavefront only (one lane per vertex), so the other
 // wavefronts issue no solve instructions.
 //
+// The lanes take the group's sub-faces in sweep order (k_sweep_order): those
+// between two cells first, so the ghost states and the second cell's loads are
+// whole wavefronts' work, and the wall faces of one-layer meshes, whose lambdas
+// stand still from the second iteration on, skip its divisions and rows
+// together.  A group whose lambdas all stand leaves the iterations.  Divisions
+// that share a divisor share its reciprocal (quot).  What bounds the sweep is
+// latency between the barriers (VALU issue 47 %, LDS 25 % of the time; four
+// wavefronts per SIMD instead of three, 15 registers spilled: no faster).  Per
+// launch, exact, first order: tri 768^2 1,142 -> 1,035 us, tets 40^3 (a blast,
+// mostly at rest) 230 -> 150 us, quad 128^2 34.6 -> 29.2 us; VALU instructions
+// per wavefront 1,547 -> 1,264.
+//
 // Output: one row of six partial sums per node-sorted sub-element slot q
 // (vertex-major, so a group's rows are one contiguous run): P[6*q + k] = sum
 // over the vertex's sub-faces of area*flux_k (k < 5) and P[6*q + 5] = sum of
@@ -79,6 +91,35 @@ SFV_DEV int seg_of(const int *tab, int n, int x) {
   return lo;
 }
 
+// One workgroup per vertex group: the sweep's copy of its sub-faces, those
+// between two cells first, the boundary ones after them, each part in order.
+static __global__ __launch_bounds__(kGrpThreads) void k_sweep_order(DevMesh m) {
+  __shared__ int vtab[kGrpVert + 1];
+  __shared__ int cnt[kGrpThreads / 64 + 1];
+  const int *gh = m.grp + kGrpHdr * (long)blockIdx.x;
+  const int vb = gh[0], nv = gh[1], sf0 = gh[2], nsf = gh[3];
+  const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63;
+  if (tid <= nv) vtab[tid] = m.sf_off[vb + tid] - sf0;
+  const bool active = tid < nsf;
+  const long s = sf0 + (active ? tid : 0);
+  const int re = m.sf_re[s];
+  const uint64_t inner = __ballot(active && re >= 0);
+  if (lane == 0) cnt[wv] = __popcll(inner);
+  __syncthreads();
+  if (!active) return;
+  int before = 0, total = 0;
+  for (int q = 0; q < kGrpThreads / 64; q++) {
+    if (q < wv) before += cnt[q];
+    total += cnt[q];
+  }
+  before += __popcll(inner & ((1ull << lane) - 1));
+  const long w = sf0 + (re >= 0 ? before : total + tid - before);
+  for (int d = 0; d < 4; d++) m.wsfn[d * m.SF + w] = m.sfn[d * m.SF + s];
+  m.ws_le[w] = m.sf_le[s];
+  m.ws_re[w] = re;
+  m.ws_id[w] = (uint16_t)(tid | seg_of(vtab, nv, tid) << 8);
+}
+
 struct FluxLds {
   double red[12][kRedStride];
   double sum[kGrpVert][9];
@@ -86,8 +127,17 @@ struct FluxLds {
   double bp[kGrpVert][3];
   int vtab[kGrpVert + 1];
   int lc[kGrpThreads];
+  int changed[10];  // nodal iteration it: some sub-face's lambda moved
   uint8_t vbound[kGrpVert];
 };
+
+// max(0, d / a) for a sound speed a with y = recip_of(a), for the factor 1 +
+// 1.5 max(0, d / a) (a quotient too small for quot's range leaves it at 1):
+// nothing to divide where d is not positive (d = 0 over a = 0 keeps its NaN)
+SFV_DEV double excess(double d, double a, double y) {
+  if (d <= 0.0 && a > 0.0) return 0.0;
+  return dmax(0.0, in_range(a, 0x1p-100, 0x1p100) && d <= 0x1p500 ? quot(d, a, y) : d / a);
+}
 
 // Nodal velocity of one vertex from its summed matrix S (6 distinct entries)
 // and right-hand side R (S[6..8]): ns_euler_rs_module.F90:406-421.
@@ -110,7 +160,7 @@ SFV_DEV void nodal_velocity(const BCParams &bc, const double *S, const double *B
       const double sc = (vn3[0] * B[0] + vn3[1] * B[1] + vn3[2] * B[2]) / (B[0] * B[0] + B[1] * B[1] + B[2] * B[2]);
       for (int d = 0; d < 3; d++) vn3[d] = vn3[d] - sc * B[d];
     } else {
-      lu_solve<3>(M, R, vn3);
+      lu_solve3(M, R, vn3);
     }
   } else {
     pinv3_sym(S, M);
@@ -128,6 +178,7 @@ SFV_DEV void node_flux_group(const FluxArgs &a, const double *__restrict__ U, in
   const int vb = gh[0], nv = gh[1], sf0 = gh[2], nsf = gh[3], se0 = gh[4], nse = gh[5];
 
   // ---- stage per-vertex data; issue the sub-face and slot loads
+  if (tid < 10) L.changed[tid] = 0;
   if (tid <= nv) L.vtab[tid] = m.sf_off[vb + tid] - sf0;
   if (tid < nv) {
     L.vbound[tid] = m.vbound[vb + tid];
@@ -138,16 +189,20 @@ SFV_DEV void node_flux_group(const FluxArgs &a, const double *__restrict__ U, in
     }
   }
   const bool active = tid < nsf;
-  // inactive threads mirror the group's first sub-face so every load is in
+  // inactive threads mirror the group's first entry so every load is in
   // bounds; their contributions are masked below
-  const long s = sf0 + (active ? tid : 0);
+  const long w = sf0 + (active ? tid : 0);
   double n[3], area;
-  n[0] = m.sfn[s];
-  n[1] = m.sfn[m.SF + s];
-  n[2] = m.sfn[2 * m.SF + s];
-  area = m.sfn[3 * m.SF + s];
-  const int le = m.sf_le[s];
-  const int re = m.sf_re[s];
+  n[0] = m.wsfn[w];
+  n[1] = m.wsfn[m.SF + w];
+  n[2] = m.wsfn[2 * m.SF + w];
+  area = m.wsfn[3 * m.SF + w];
+  const int le = m.ws_le[w];
+  const int re = m.ws_re[w];
+  const int id = m.ws_id[w];
+  const int lid = active ? id & 0xFF : tid;  // its place in the LDS rows
+  const int vl = id >> 8;
+  const long s = sf0 + (id & 0xFF);
   const bool has_slot = tid < nse;
   uint32_t src = 0xFFFFFFFFu;
   int slot_cell = -1;
@@ -156,7 +211,6 @@ SFV_DEV void node_flux_group(const FluxArgs &a, const double *__restrict__ U, in
     slot_cell = m.se_cell[se0 + tid];
   }
   __syncthreads();
-  const int vl = seg_of(L.vtab, nv, tid);
   const int v = vb + vl;
 
   // ---- left/right primitive states (reconstruct_lr_w)
@@ -219,21 +273,24 @@ SFV_DEV void node_flux_group(const FluxArgs &a, const double *__restrict__ U, in
     const double rhor = wr[0], pr = wr[4], ar = ar_cached ? ar_c : sound_speed(wr);
     const double vn_l = wl[1] * n[0] + wl[2] * n[1] + wl[3] * n[2];
     const double vn_r = wr[1] * n[0] + wr[2] * n[1] + wr[3] * n[2];
+    const double yal = recip_of(al), yar = recip_of(ar);
     for (int iter = 1; iter <= 4; iter++) {
+      const double l0 = lam_l, r0 = lam_r;
+      double vs = vbar;
       if (iter == 1) {
         lam_l = dmax(dmax(dmax(lam_l, al * rhol), sqrt(rhol * dmax(0.0, pr - pl))), -rhol * (vn_r - vn_l));
         lam_r = dmax(dmax(dmax(lam_r, ar * rhor), sqrt(rhor * dmax(0.0, pl - pr))), -rhor * (vn_r - vn_l));
-        vbar = (lam_l * vn_l + lam_r * vn_r - (pr - pl)) / (lam_r + lam_l);
-        lam_l = dmax(lam_l, al * rhol * (1.0 + 1.5 * dmax(0.0, -(vbar - vn_l) / al)));
-        lam_r = dmax(lam_r, ar * rhor * (1.0 + 1.5 * dmax(0.0, (vbar - vn_r) / ar)));
-      } else if (wall && bc.bc_style == 1) {
-        lam_l = dmax(lam_l, al * rhol * (1.0 + 1.5 * dmax(0.0, -(vbar - vn_l) / al)));
-        lam_r = dmax(lam_r, ar * rhor * (1.0 + 1.5 * dmax(0.0, (vbar - vn_r) / ar)));
-      } else {
-        double v_et = v_node[0] * n[0] + v_node[1] * n[1] + v_node[2] * n[2];
-        lam_l = dmax(lam_l, al * rhol * (1.0 + 1.5 * dmax(0.0, -(v_et - vn_l) / al)));
-        lam_r = dmax(lam_r, ar * rhor * (1.0 + 1.5 * dmax(0.0, (v_et - vn_r) / ar)));
+        vs = (lam_l * vn_l + lam_r * vn_r - (pr - pl)) / (lam_r + lam_l);
+      } else if (!(wall && bc.bc_style == 1)) {
+        vs = v_node[0] * n[0] + v_node[1] * n[1] + v_node[2] * n[2];
       }
+      lam_l = dmax(lam_l, al * rhol * (1.0 + 1.5 * excess(-(vs - vn_l), al, yal)));
+      lam_r = dmax(lam_r, ar * rhor * (1.0 + 1.5 * excess(vs - vn_r, ar, yar)));
+      // vbar, the nodal contributions and so the nodal velocity follow from the
+      // lambdas alone: where none moved the rows stand, and a group where none
+      // moved has reached the fixed point that further iterations would repeat
+      const bool moved = iter == 1 || !(lam_l == l0 && lam_r == r0);
+      if (moved) {
       vbar = (lam_l * vn_l + lam_r * vn_r - (pr - pl)) / (lam_r + lam_l);
       // contributions to the nodal matrix (6 distinct entries) and Rp
       double cm = iso ? (lam_r + lam_l) : (lam_r + lam_l) * area;
@@ -250,16 +307,19 @@ SFV_DEV void node_flux_group(const FluxArgs &a, const double *__restrict__ U, in
         }
       }
       if (!active || excl) addm = addr = false;
-      L.red[0][tid] = addm ? cm * (n[0] * n[0]) : 0.0;
-      L.red[1][tid] = addm ? cm * (n[0] * n[1]) : 0.0;
-      L.red[2][tid] = addm ? cm * (n[0] * n[2]) : 0.0;
-      L.red[3][tid] = addm ? cm * (n[1] * n[1]) : 0.0;
-      L.red[4][tid] = addm ? cm * (n[1] * n[2]) : 0.0;
-      L.red[5][tid] = addm ? cm * (n[2] * n[2]) : 0.0;
-      L.red[6][tid] = addr ? cr * n[0] : 0.0;
-      L.red[7][tid] = addr ? cr * n[1] : 0.0;
-      L.red[8][tid] = addr ? cr * n[2] : 0.0;
+      L.red[0][lid] = addm ? cm * (n[0] * n[0]) : 0.0;
+      L.red[1][lid] = addm ? cm * (n[0] * n[1]) : 0.0;
+      L.red[2][lid] = addm ? cm * (n[0] * n[2]) : 0.0;
+      L.red[3][lid] = addm ? cm * (n[1] * n[1]) : 0.0;
+      L.red[4][lid] = addm ? cm * (n[1] * n[2]) : 0.0;
+      L.red[5][lid] = addm ? cm * (n[2] * n[2]) : 0.0;
+      L.red[6][lid] = addr ? cr * n[0] : 0.0;
+      L.red[7][lid] = addr ? cr * n[1] : 0.0;
+      L.red[8][lid] = addr ? cr * n[2] : 0.0;
+      }
+      if (active && moved) L.changed[iter - 1] = 1;
       __syncthreads();
+      if (!L.changed[iter - 1]) break;  // uniform
       for (int p = tid; p < nv * 9; p += kGrpThreads) {
         const int vv = p / 9, c = p - vv * 9;
         L.sum[vv][c] = seg_sum(L.red[c], L.vtab[vv], L.vtab[vv + 1]);
@@ -280,7 +340,7 @@ SFV_DEV void node_flux_group(const FluxArgs &a, const double *__restrict__ U, in
       for (int d = 0; d < 3; d++) a.vp[d * m.V + vb + tid] = L.vn[tid][d];
     if (iso) {
       // warea = minval(area)/area over the vertex's sub-faces
-      L.red[0][tid] = active ? area : 1e300;
+      L.red[0][lid] = active ? area : 1e300;
       __syncthreads();
       if (tid < nv) {
         double mn = L.red[0][L.vtab[tid]];
@@ -297,19 +357,19 @@ SFV_DEV void node_flux_group(const FluxArgs &a, const double *__restrict__ U, in
     const double vn_r = wr[1] * n[0] + wr[2] * n[1] + wr[3] * n[2];
     const bool w1 = (bc.bc_style == 1 && wall);
     for (int iter = 1; iter <= 10; iter++) {
+      const double l0 = lam_l, r0 = lam_r;
+      double ps = vbar;
       if (iter == 1) {
         lam_l = dmax(dmax(dmax(lam_l, al * rhol), sqrt(rhol * dmax(0.0, pr - pl))), -rhol * (vn_r - vn_l));
         lam_r = dmax(dmax(dmax(lam_r, ar * rhor), sqrt(rhor * dmax(0.0, pl - pr))), -rhor * (vn_r - vn_l));
-        vbar = (lam_r * pl + lam_l * pr - lam_r * lam_l * (vn_r - vn_l)) / (lam_r + lam_l);
-        lam_l = dmax(lam_l, al * rhol + 1.5 * sqrt(dmax(0.0, (vbar - pl) * rhol)));
-        lam_r = dmax(lam_r, ar * rhor + 1.5 * sqrt(dmax(0.0, (vbar - pr) * rhor)));
-      } else if (w1) {
-        lam_l = dmax(lam_l, al * rhol + 1.5 * sqrt(dmax(0.0, (vbar - pl) * rhol)));
-        lam_r = dmax(lam_r, ar * rhor + 1.5 * sqrt(dmax(0.0, (vbar - pr) * rhor)));
-      } else {
-        lam_l = dmax(lam_l, al * rhol + 1.5 * sqrt(dmax(0.0, (p_nodal - pl) * rhol)));
-        lam_r = dmax(lam_r, ar * rhor + 1.5 * sqrt(dmax(0.0, (p_nodal - pr) * rhor)));
+        ps = (lam_r * pl + lam_l * pr - lam_r * lam_l * (vn_r - vn_l)) / (lam_r + lam_l);
+      } else if (!w1) {
+        ps = p_nodal;
       }
+      lam_l = dmax(lam_l, al * rhol + 1.5 * sqrt(dmax(0.0, (ps - pl) * rhol)));
+      lam_r = dmax(lam_r, ar * rhor + 1.5 * sqrt(dmax(0.0, (ps - pr) * rhor)));
+      const bool moved = iter == 1 || !(lam_l == l0 && lam_r == r0);  // as above
+      if (moved) {
       vbar = (lam_r * pl + lam_l * pr - lam_r * lam_l * (vn_r - vn_l)) / (lam_r + lam_l);
       double c1, c2;
       if (w1) {
@@ -319,9 +379,12 @@ SFV_DEV void node_flux_group(const FluxArgs &a, const double *__restrict__ U, in
         c1 = (1.0 / lam_r + 1.0 / lam_l) * area * vbar;
         c2 = (1.0 / lam_r + 1.0 / lam_l) * area;
       }
-      L.red[0][tid] = active ? c1 : 0.0;
-      L.red[1][tid] = active ? c2 : 0.0;
+      L.red[0][lid] = active ? c1 : 0.0;
+      L.red[1][lid] = active ? c2 : 0.0;
+      }
+      if (active && moved) L.changed[iter - 1] = 1;
       __syncthreads();
+      if (!L.changed[iter - 1]) break;  // uniform
       if (tid < nv) {
         const double s1 = seg_sum(L.red[0], L.vtab[tid], L.vtab[tid + 1]);
         const double s2 = seg_sum(L.red[1], L.vtab[tid], L.vtab[tid + 1]);
@@ -339,7 +402,20 @@ SFV_DEV void node_flux_group(const FluxArgs &a, const double *__restrict__ U, in
       flux_two_wave(wl, wr, n, fx, sl, sr);
     } else {
       double vn = wall ? 0.0 : (v_node[0] * n[0] + v_node[1] * n[1] + v_node[2] * n[2]);
-      bool ok = flux_multi_point(wl, wr, n, fx, vn, lam_l, lam_r, sl, sr);
+      bool ok;
+      // multi_point: straight into the rows (free since the last iteration's
+      // barrier), so the ten fluxes are never held together
+      auto emit = [&](int k, double xl, double xr) {
+        if (SCHEME == kMultiPoint) {
+          L.red[k][lid] = area * xl;
+          L.red[6 + k][lid] = area * xr;
+        } else {
+          fx[k] = xl;
+          fx[5 + k] = xr;
+        }
+      };
+      if (!flux_multi_point_q(wl, wr, n, emit, vn, lam_l, lam_r, sl, sr, ok))
+        ok = flux_multi_point(wl, wr, n, emit, vn, lam_l, lam_r, sl, sr);
       if (!ok && active) atomicOr(a.err, (int)kErrNegStarDensity);
     }
     if (SCHEME == kMultiPointIso) {
@@ -360,13 +436,14 @@ SFV_DEV void node_flux_group(const FluxArgs &a, const double *__restrict__ U, in
   }
 
   // ---- area*flux per sub-element slot (ns_euler_module.F90:506-517)
-  for (int k = 0; k < 5; k++) {
-    L.red[k][tid] = area * fx[k];
-    L.red[6 + k][tid] = area * fx[5 + k];
-  }
-  L.red[5][tid] = area * dmax(0.0, -sl);
-  L.red[11][tid] = area * dmax(0.0, sr);
-  L.lc[tid] = le;
+  if (SCHEME != kMultiPoint || excl)
+    for (int k = 0; k < 5; k++) {
+      L.red[k][lid] = area * fx[k];
+      L.red[6 + k][lid] = area * fx[5 + k];
+    }
+  L.red[5][lid] = area * dmax(0.0, -sl);
+  L.red[11][lid] = area * dmax(0.0, sr);
+  L.lc[lid] = le;
   __syncthreads();
   if (has_slot) {
     double acc[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};

@@ -45,6 +45,25 @@ struct BCParams {
 SFV_DEV double dmax(double a, double b) { return a > b ? a : b; }
 SFV_DEV double dmin(double a, double b) { return a < b ? a : b; }
 
+// Quotients by a divisor that several numerators share.  A compiled FP64
+// division is the refined reciprocal (v_rcp_f64 and two Newton steps), the
+// product, one residual correction, and v_div_scale / v_div_fixup around them
+// for extreme exponents, which leave operands of ordinary exponents alone.  So
+// the reciprocal formed once and the last three operations per numerator give
+// the bits of a / b in 3 instructions instead of 11, for b within 2^+-400, a
+// within 2^+-500 or zero (the sign of a zero quotient aside); the callers check
+// the ranges and divide where they do not hold.
+SFV_DEV double recip_of(double b) {
+  const double y0 = __builtin_amdgcn_rcp(b);
+  const double y1 = __builtin_fma(y0, __builtin_fma(-b, y0, 1.0), y0);
+  return __builtin_fma(y1, __builtin_fma(-b, y1, 1.0), y1);
+}
+SFV_DEV double quot(double a, double b, double y) {
+  const double q = a * y;
+  return __builtin_fma(__builtin_fma(-b, q, a), y, q);
+}
+SFV_DEV bool in_range(double a, double lo, double hi) { return a >= lo && a <= hi; }
+
 // conserv_to_primit / primit_to_conserv, ns_euler_primitives_module.F90:7-31
 SFV_DEV void to_prim(const double *u, double *w) {
   w[0] = u[0];
@@ -278,8 +297,10 @@ SFV_DEV void flux_three_wave(const double *wl, const double *wr, const double *n
 }
 
 // multi_point, ns_euler_rs_module.F90:200-286.  Returns false on a negative
-// star density (the reference stops there).
-SFV_DEV bool flux_multi_point(const double *wl, const double *wr, const double *n, double *out, double v_et,
+// star density (the reference stops there).  emit(k, left, right) takes component
+// k of both sides' fluxes.
+template <class Emit>
+SFV_DEV bool flux_multi_point(const double *wl, const double *wr, const double *n, Emit emit, double v_et,
                               double ll, double lr, double &sl, double &sr) {
   Side L, R;
   side(wl, n, L, false);
@@ -303,10 +324,73 @@ SFV_DEV bool flux_multi_point(const double *wl, const double *wr, const double *
   for (int k = 0; k < 5; k++) {
     double c = 0.5 * (L.f[k] + R.f[k]) -
                0.5 * (fabs(sl) * (ql[k] - L.u[k]) + fabs(v_et) * (qr[k] - ql[k]) + fabs(sr) * (R.u[k] - qr[k]));
-    out[k] = c - 0.5 * (pr_bar - pl_bar) * e[k];
-    out[5 + k] = -(c + 0.5 * (pr_bar - pl_bar) * e[k]);
+    emit(k, c - 0.5 * (pr_bar - pl_bar) * e[k], -(c + 0.5 * (pr_bar - pl_bar) * e[k]));
   }
   return !(rl < 0.0 || rr < 0.0);
+}
+
+// The same with shared reciprocals: ok is false where an operand leaves the
+// ranges in which the quotients are those of the divisions above (the caller
+// then takes flux_multi_point).  A small (v_et - vn) or pressure-work numerator
+// needs no lower bound: its quotient is added to 1/rho or e, more than 2^300
+// larger, and leaves them as they are either way.
+SFV_DEV bool side_q(const double *w, const double *n, double yg, double vn, double lam, double v_et, double sg,
+                    Side &s, double &rstar, double &pbar, double &estar, double &wave) {
+  s.rho = w[0];
+  s.vn = vn;
+  s.p = w[4];
+  s.u[0] = w[0];
+  s.u[1] = w[1] * w[0];
+  s.u[2] = w[2] * w[0];
+  s.u[3] = w[3] * w[0];
+  s.u[4] = quot(w[4], kGm1, yg) + 0.5 * w[0] * (w[1] * w[1] + w[2] * w[2] + w[3] * w[3]);
+  const double yr = recip_of(s.rho), yl = recip_of(lam);
+  s.e = quot(s.u[4], s.rho, yr);
+  s.f[0] = s.vn * s.u[0];
+  for (int d = 0; d < 3; d++) s.f[1 + d] = s.vn * s.u[1 + d] + s.p * n[d];
+  s.f[4] = (s.u[4] + s.p) * s.vn;
+  // left (sg = 1): 1/(1/rho + (v_et - vn)/lam), p - lam (v_et - vn); right (sg =
+  // -1): 1/(1/rho + (vn - v_et)/lam), p + lam (v_et - vn)
+  const double dv = v_et - s.vn, da = sg > 0.0 ? dv : s.vn - v_et;
+  const double x = quot(1.0, s.rho, yr) + quot(da, lam, yl);
+  rstar = quot(1.0, x, recip_of(x));
+  pbar = sg > 0.0 ? s.p - lam * dv : s.p + lam * dv;
+  const double work = sg > 0.0 ? s.p * s.vn - pbar * v_et : pbar * v_et - s.p * s.vn;
+  estar = s.e + quot(work, lam, yl);
+  wave = quot(lam, s.rho, yr);
+  return in_range(s.rho, 0x1p-100, 0x1p100) && in_range(lam, 0x1p-200, 0x1p200) && in_range(s.p, 0x1p-300, 0x1p200) &&
+         in_range(fabs(x), 0x1p-150, 0x1p150) && fabs(s.vn) <= 0x1p100 && s.u[4] <= 0x1p300;
+}
+template <class Emit>
+SFV_DEV bool flux_multi_point_q(const double *wl, const double *wr, const double *n, Emit emit, double v_et,
+                                double ll, double lr, double &sl, double &sr, bool &pos) {
+  Side L, R;
+  double g = kGm1;
+  asm("" : "+v"(g));  // the reciprocal of the division the hardware would do, not a folded one
+  const double yg = recip_of(g);
+  double rl, rr, pl_bar, pr_bar, el, er, al, ar;
+  const double vnl = wl[1] * n[0] + wl[2] * n[1] + wl[3] * n[2], vnr = wr[1] * n[0] + wr[2] * n[1] + wr[3] * n[2];
+  const bool okl = side_q(wl, n, yg, vnl, ll, v_et, 1.0, L, rl, pl_bar, el, al);
+  const bool okr = side_q(wr, n, yg, vnr, lr, v_et, -1.0, R, rr, pr_bar, er, ar);
+  double ql[5], qr[5];
+  ql[0] = rl;
+  qr[0] = rr;
+  for (int d = 0; d < 3; d++) {
+    ql[1 + d] = rl * (wl[1 + d] + (v_et - L.vn) * n[d]);
+    qr[1 + d] = rr * (wr[1 + d] + (v_et - R.vn) * n[d]);
+  }
+  ql[4] = rl * el;
+  qr[4] = rr * er;
+  sl = L.vn - al;
+  sr = R.vn + ar;
+  const double e[5] = {0.0, n[0], n[1], n[2], v_et};
+  for (int k = 0; k < 5; k++) {
+    double c = 0.5 * (L.f[k] + R.f[k]) -
+               0.5 * (fabs(sl) * (ql[k] - L.u[k]) + fabs(v_et) * (qr[k] - ql[k]) + fabs(sr) * (R.u[k] - qr[k]));
+    emit(k, c - 0.5 * (pr_bar - pl_bar) * e[k], -(c + 0.5 * (pr_bar - pl_bar) * e[k]));
+  }
+  pos = !(rl < 0.0 || rr < 0.0);
+  return okl && okr && fabs(v_et) <= 0x1p100;
 }
 
 // multi_point_pressure (:555-616) and _ph (:618-679)
@@ -425,6 +509,69 @@ SFV_DEV void lu_solve(double *A, const double *b, double *x) {
     }
 #pragma unroll
   for (int i = 0; i < N; i++) x[i] = w[i];
+}
+
+// lu_solve<3> with each pivot's reciprocal formed once, for the scaling of L and
+// for the back substitution (a shorter chain: the solve is one lane per vertex
+// while the workgroup waits).  Leaves the ranges of quot: lu_solve<3>.
+SFV_DEV void lu_solve3(const double *M, const double *b, double *x) {
+  double A[9], w[3], y[3];
+  for (int i = 0; i < 9; i++) A[i] = M[i];
+  for (int i = 0; i < 3; i++) w[i] = b[i];
+  bool ok = true;
+#pragma unroll
+  for (int k = 0; k < 3; k++) {
+    int p = k;
+    double amax = fabs(A[k + 3 * k]);
+#pragma unroll
+    for (int i = k + 1; i < 3; i++)
+      if (fabs(A[i + 3 * k]) > amax) {
+        amax = fabs(A[i + 3 * k]);
+        p = i;
+      }
+#pragma unroll
+    for (int i = k + 1; i < 3; i++)
+      if (i == p) {
+#pragma unroll
+        for (int j = 0; j < 3; j++) {
+          const double t = A[k + 3 * j];
+          A[k + 3 * j] = A[i + 3 * j];
+          A[i + 3 * j] = t;
+        }
+        const double t = w[k];
+        w[k] = w[i];
+        w[i] = t;
+      }
+    ok = ok && in_range(amax, 0x1p-400, 0x1p400);
+    y[k] = recip_of(A[k + 3 * k]);
+    if (k < 2) {
+      const double r = quot(1.0, A[k + 3 * k], y[k]);
+#pragma unroll
+      for (int i = k + 1; i < 3; i++) A[i + 3 * k] = A[i + 3 * k] * r;
+    }
+#pragma unroll
+    for (int j = k + 1; j < 3; j++)
+#pragma unroll
+      for (int i = k + 1; i < 3; i++) A[i + 3 * j] = A[i + 3 * j] - A[i + 3 * k] * A[k + 3 * j];
+  }
+#pragma unroll
+  for (int k = 0; k < 3; k++)
+    if (w[k] != 0.0)
+#pragma unroll
+      for (int i = k + 1; i < 3; i++) w[i] = w[i] - w[k] * A[i + 3 * k];
+#pragma unroll
+  for (int k = 2; k >= 0; k--)
+    if (w[k] != 0.0) {
+      ok = ok && in_range(fabs(w[k]), 0x1p-500, 0x1p500);
+      w[k] = quot(w[k], A[k + 3 * k], y[k]);
+#pragma unroll
+      for (int i = 0; i < k; i++) w[i] = w[i] - w[k] * A[i + 3 * k];
+    }
+  if (!ok) {
+    for (int i = 0; i < 9; i++) A[i] = M[i];
+    lu_solve<3>(A, b, w);
+  }
+  for (int i = 0; i < 3; i++) x[i] = w[i];
 }
 
 // Cofactor inverse of the 3x3 matrix with rows (a b c), (d e f), (g h i),

@@ -84,6 +84,39 @@ def test_euler_flux_first_order_bit_exact(solver, name, scheme):
         assert np.array_equal(vp, r_vp), np.abs(vp - r_vp).max()
 
 
+# (exponent of rho, exponent of p, exponent of the velocities): the shared
+# reciprocals of the node sweep hold in a range of exponents and give way to
+# plain divisions outside it; each side of those limits, velocities so small
+# that quotients leave the normal range, and a state at rest, whose nodal
+# iterations reach their fixed point at once
+RANGES = [(0, 0, 0), (-99, -99, 0), (-101, -101, 0), (99, 99, 0), (120, 120, 0), (0, -299, -160), (0, -310, -160),
+          (0, 0, -480), (0, 0, -520), (0, 0, -905), (0, 0, -960), (0, 0, -1020), (0, 0, None)]
+
+
+@pytest.mark.parametrize("name", ["quad8lr", "tri7", "tet3"])
+@pytest.mark.parametrize("er,ep,ev", RANGES)
+def test_euler_flux_extreme_exponents_bit_exact(solver, name, er, ep, ev):
+    print(f"[gpu] flux ranges {name} {er} {ep} {ev}", flush=True)
+    mesh, om = _pair(solver, name)
+    kw = dict(boundary_2d=mesh.boundary_2d, bcs=[("wall", (0,) * 5)] * len(_bcs_for(name)))
+    solver.set_config(make_config("multi_point", **kw))
+    cfg = O.make_config("multi_point", **kw)
+    w = np.zeros((om.n_elems, 5))
+    rng = np.random.default_rng(21)
+    w[:, 0] = (1.0 + 0.3 * rng.random(om.n_elems)) * 2.0 ** er
+    w[:, 4] = (1.0 + (0.0 if ev is None else 0.3) * rng.random(om.n_elems)) * 2.0 ** ep
+    if ev is not None:
+        w[:, 1:4] = rng.uniform(-0.4, 0.4, (om.n_elems, 3)) * 2.0 ** ev
+        if ev < 0:
+            w[:, 4] = 2.0 ** ep  # the velocities alone drive the fluxes
+    sol = mg.primit_to_conserv(w)
+    rhs, sl, vp = solver.compute_euler_flux(sol, want_vp=True)
+    r_rhs, r_sl, r_vp = om.compute_euler_flux(cfg, sol, want_vp=True)
+    assert np.array_equal(rhs, r_rhs, equal_nan=True), np.abs(rhs - r_rhs).max()
+    assert np.array_equal(sl, r_sl, equal_nan=True)
+    assert np.array_equal(vp, r_vp, equal_nan=True)
+
+
 @pytest.mark.parametrize("bc_style", [0, 1, 2])
 @pytest.mark.parametrize("excl", [False, True])
 def test_multi_point_bc_styles_bit_exact(solver, bc_style, excl):
