@@ -147,7 +147,7 @@ struct subfv_ctx {
   double *dblk = nullptr;      // [C][kDiffBlk] the cells' viscous blocks
   double *mu_cell = nullptr, *mu_blk = nullptr;  // Sutherland: [C] viscosities; block minima + mu0corr
   int diff_cls = 0;  // DiffClass of the mesh
-  int diff_nim = 0, diff_nfm = 0, diff_nsm = 0, diff_lmat = 0;  // a vertex's largest sizes (DiffArgs)
+  int diff_nim = 0, diff_nfm = 0, diff_nsm = 0, diff_lds = 0;  // a vertex's largest sizes (DiffArgs)
   long pre_n = 0;  // doubles in the packed inverses
   int *derr = nullptr;  // [2]: error bits of the path, failed check_mesh cells
   StepState *st = nullptr;
@@ -699,7 +699,7 @@ DiffArgs diff_args(subfv_ctx *c) {
   a.nim = c->diff_nim;
   a.nfm = c->diff_nfm;
   a.nsm = c->diff_nsm;
-  a.lmat = c->diff_lmat;
+  a.lds_wave = c->diff_lds;
   a.parts = 3;
   return a;
 }
@@ -757,15 +757,25 @@ int ensure_diffusion(subfv_ctx *c) {
     // reserves all (its inverses for cell viscosities are stored too)
     std::vector<uint64_t> off(h.nv);
     uint64_t at = 0;
-    int lmat = 1;
     for (int v = 0; v < h.nv; v++) {
       const uint64_t ni = st[v] & 0xFF, tag = st[v] >> 8;
       const uint64_t nb = tag || c->diff_cls == kDiffLarge ? ni * ni : ni * (ni + 1) / 2;
       off[v] = at | ni << 48 | tag << 56;
-      lmat = std::max(lmat, (int)(10 * nb));
       at += 10 * nb;
     }
-    c->diff_lmat = lmat;
+    c->diff_lds = 0;
+    if (c->diff_cls != kDiffLarge) {
+      const int per = kDiffApplyVerts[c->diff_cls];
+      for (int v0 = 0; v0 < h.nv; v0 += per) {
+        int sum = 0;
+        // past the last vertex the lanes mirror it
+        for (int k = 0; k < per; k++) {
+          const int v = std::min(v0 + k, h.nv - 1);
+          sum += diff_apply_lds(st[v] & 0xFF, h.sf_off[v + 1] - h.sf_off[v]);
+        }
+        c->diff_lds = std::max(c->diff_lds, sum);
+      }
+    }
     if ((r = room(fixed + sizeof(double) * at))) return r;
     if ((r = upload(c, &c->doff, off))) return r;
     if ((r = dalloc(c, &c->pre, (size_t)at))) return r;

@@ -189,12 +189,14 @@ struct SlotReg {
   double g[kSlotSrc][3], gh[kSlotSrc];
 };
 
+template <bool VAR>
 SFV_DEV void slot_load(const DiffArgs &a, int q, SlotReg &r, double mu0) {
   const long cell = a.m.se_cell[q];
   r.code = (int)a.scode[q];
   r.ivol = a.sivol[q];
-  r.mu = a.mu_cell ? a.mu_cell[cell] : a.p.mu;
-  r.kv = (a.mu_cell ? r.mu * a.p.cv * kGamma / a.p.pr : a.p.kap) * r.ivol;  // kappa (ns_diffusion_module.F90:186-194)
+  r.mu = VAR && a.mu_cell ? a.mu_cell[cell] : a.p.mu;
+  // kappa (ns_diffusion_module.F90:186-194)
+  r.kv = (VAR && a.mu_cell ? r.mu * a.p.cv * kGamma / a.p.pr : a.p.kap) * r.ivol;
   r.c2 = r.mu - mu0;
   r.c3 = mu0 - (2.0 / 3.0) * r.mu;
   double u[5];
@@ -534,7 +536,7 @@ __global__ __launch_bounds__(64) void k_visc(DiffArgs a) {
   const double mu0 = a.mu_cell ? *a.mu_min : a.p.mu0;
   // ---- (a)
   SlotReg r;
-  if (lane < 4 * ns) slot_load(a, se0 + (lane >> 2), r, mu0);
+  if (lane < 4 * ns) slot_load<true>(a, se0 + (lane >> 2), r, mu0);
   bool walls = false;
   for (int l = lane; l < nf; l += LPV) {
     const long s = sf0 + l;
@@ -596,14 +598,15 @@ __global__ __launch_bounds__(64) void k_visc(DiffArgs a) {
     }
   }
   if (MODE == kStore && live) {
+    // value k of block q at pre[k nb + q], k = 9 the heat system's entry
     const bool half = !tag;
-    const int nm = mom_size(half, ni);
+    const int nb = half ? tri(ni) : ni * ni;
     for (int q = lane; q < ni * ni; q += LPV) {
       const int pe = q / ni, po = q - pe * ni;
       if (half && po > pe) continue;
-      const int at = half ? 9 * (tri(pe) + po) : 9 * q;
-      for (int k = 0; k < 9; k++) pre[at + k] = Lm[9 * q + k];
-      pre[nm + heat_at(half, ni, pe, po)] = Lh[q];
+      double *out = pre + (half ? tri(pe) + po : q);
+      for (int k = 0; k < 9; k++) out[k * nb] = Lm[9 * q + k];
+      out[9 * nb] = Lh[q];
     }
   }
   const double *const Gm = MODE == kGlobal ? pre : Lm;
@@ -611,7 +614,7 @@ __global__ __launch_bounds__(64) void k_visc(DiffArgs a) {
   // ---- (b)
   const int rounds = (4 * ns + LPV - 1) / LPV;
   for (int t = lane; t < 4 * ns; t += LPV) {
-    if (t != lane) slot_load(a, se0 + (t >> 2), r, mu0);
+    if (t != lane) slot_load<true>(a, se0 + (t >> 2), r, mu0);
     slot_faces(A, r);
     slot_fluxes<FORM || MODE == kGlobal>(A, ty, t & 3, r);
     if ((t & 3) == 0)
@@ -659,7 +662,7 @@ __global__ __launch_bounds__(64) void k_visc(DiffArgs a) {
   for (int t = lane; t < 4 * ns; t += LPV) {
     const int f = t & 3;
     if (rounds > 1) {
-      slot_load(a, se0 + (t >> 2), r, mu0);
+      slot_load<true>(a, se0 + (t >> 2), r, mu0);
       slot_faces(A, r);
       slot_fluxes<FORM || MODE == kGlobal>(A, ty, f, r);
     }
@@ -732,16 +735,39 @@ __global__ __launch_bounds__(64) void k_visc(DiffArgs a) {
 
 // The scatter terms of every slot with a constant viscosity: rhs rows of four
 // partials (rho u, rho v, rho w without the block's own-cell part; E), one lane
-// per slot and row.  GLOBAL: the inverses are read in place (large class), else
-// staged in LDS.
-// 16 lanes per vertex (four vertices per wavefront) since a prism vertex has 6
-// slots, 12 faces and 18 rows.  On tri 1024^2 (2.1M prisms and vertices) the
-// stored products took 4.88 ms per residual at 4.6 TB/s (19 GB); the inverses
-// (4 GB) take 2.66 ms: what bounds it now is instruction issue and latency, the
-// bytes alone would take about 1.1 ms.
+// per slot.  16 lanes per vertex (four vertices per wavefront) on prism and quad
+// meshes: a prism vertex has 6 slots, 12 faces and 21 blocks.
+// The face values v = N^-1 f: a lane owns whole blocks (the first kHold of them
+// loaded at the start, in flight while the slots are read), forms their products
+// with the two faces they couple, and the products meet in LDS, where each row
+// sums its own in face order.  LDS holds the products only, sized per wavefront
+// for the vertices it has.
+// GLOBAL (large class): one lane per row reads its blocks in place.
+// On tri 1024^2 (2.1M prisms and vertices) the stored products of the dense
+// matrices took 4.88 ms per residual (19 GB, 4.6 TB/s); the inverses (4 GB)
+// staged in LDS, 9 wavefronts per CU, 2.66 ms; like this 1.46 ms, bound by
+// instruction issue (0.8 ms of it) and latency, 3.4 TB/s.
+template <bool GLOBAL>
+SFV_DEV __host__ int apply_lds(int ni, int nf) {
+  const int part = GLOBAL ? 8 * ni : (ni > 2 ? 4 * ni * ni : 8 * ni);
+  return (part + 4 * ni + 3 * nf + (ni + 1) / 2 + 1) & ~1;  // even: rows of four are read and written in pairs
+}
+SFV_DEV void put4(double *p, double a, double b, double c, double d) {
+  ((double2 *)p)[0] = make_double2(a, b);
+  ((double2 *)p)[1] = make_double2(c, d);
+}
+SFV_DEV void get4(const double *p, double *o) {
+  const double2 a = ((const double2 *)p)[0], b = ((const double2 *)p)[1];
+  o[0] = a.x;
+  o[1] = a.y;
+  o[2] = b.x;
+  o[3] = b.y;
+}
+
 template <int LPV, bool GLOBAL>
-__global__ __launch_bounds__(256, 4) void k_visc_apply(DiffArgs a) {
+__global__ __launch_bounds__(256, 3) void k_visc_apply(DiffArgs a) {
   extern __shared__ double lds_all[];
+  constexpr int kHold = GLOBAL ? 0 : 2;
   const DevMesh &m = a.m;
   const int lb = xcd_block(a.vper_xcd);  // neighbouring vertices share cells
   if (lb >= a.vblocks) return;
@@ -749,10 +775,6 @@ __global__ __launch_bounds__(256, 4) void k_visc_apply(DiffArgs a) {
   const long v_ = (long)lb * (blockDim.x / LPV) + grp;
   const bool live = v_ < m.V;
   const long v = live ? v_ : m.V - 1;  // spare lanes mirror the last vertex and store nothing
-  double *const L = lds_all + (long)grp * a.lds_stride;
-  const Lay o = lds_layout(a.lmat, a.nim, a.nfm, a.nsm, false);
-  double *const A = L + o.A, *const fL = L + o.fL, *const fh = L + o.fh, *const fv = L + o.fv, *const fhv = L + o.fhv;
-  int *const ty = (int *)(L + o.ty);
   const int sf0 = m.sf_off[v], nf = m.sf_off[v + 1] - sf0;
   const int se0 = m.se_off[v], ns = m.se_off[v + 1] - se0;
   const uint64_t dd = a.doff[v];
@@ -760,8 +782,29 @@ __global__ __launch_bounds__(256, 4) void k_visc_apply(DiffArgs a) {
   const bool tag = dd >> 56 & 1, sym = !tag;
   const double *const pre = a.pre + (dd & 0xFFFFFFFFFFFFull);
   const double mu0 = a.p.mu0;
+  const int nb = sym ? tri(ni) : ni * ni;
+  double x[kHold ? kHold : 1][10];
+#pragma unroll
+  for (int h = 0; h < kHold; h++)
+    if (lane + h * LPV < nb)
+#pragma unroll
+      for (int k = 0; k < 10; k++) x[h][k] = pre[k * nb + lane + h * LPV];
   SlotReg r;
-  if (lane < ns) slot_load(a, se0 + lane, r, mu0);
+  if (lane < ns) slot_load<false>(a, se0 + lane, r, mu0);
+  // this vertex's LDS, behind those of the wavefront's earlier vertices
+  double *L = lds_all + (long)(threadIdx.x >> 6) * a.lds_stride;
+  {
+    const int size = apply_lds<GLOBAL>(ni, nf);
+    const int mine = (threadIdx.x & 63) / LPV;
+    for (int q = 0; q < 64 / LPV - 1; q++) {
+      const int sq = __shfl(size, q * LPV);
+      if (q < mine) L += sq;
+    }
+  }
+  double *const fL = L;  // [ni][2][4] one-sided fluxes, then the block products [ni][ni][4]
+  double *const fv = L + (GLOBAL ? 8 * ni : (ni > 2 ? 4 * ni * ni : 8 * ni));  // [ni][4] rhs, then the face values
+  double *const A = fv + 4 * ni;
+  int *const ty = (int *)(A + 3 * nf);
   for (int l = lane; l < nf; l += LPV) {
     const long s = sf0 + l;
     const int fp = a.fpos[s], pos = fp & kPosMask;
@@ -769,72 +812,104 @@ __global__ __launch_bounds__(256, 4) void k_visc_apply(DiffArgs a) {
     for (int d = 0; d < 3; d++) A[3 * pos + d] = m.sfn[d * m.SF + s] * ar;
     if (pos < ni) {
       ty[pos] = face_type(a, fp, s);
-      if (fp & kPosBound) {
-        for (int d = 0; d < 3; d++) fL[6 * pos + 3 + d] = 0.0;
-        fh[2 * pos + 1] = 0.0;
-      }
-    }
-  }
-  if (!GLOBAL) {
-    const int nm = mom_size(sym, ni) + (sym ? tri(ni) : ni * ni);
-    for (int t0 = lane; t0 < nm; t0 += 8 * LPV) {
-      double x[8];
-#pragma unroll
-      for (int u = 0; u < 8; u++) x[u] = t0 + u * LPV < nm ? pre[t0 + u * LPV] : 0.0;
-#pragma unroll
-      for (int u = 0; u < 8; u++)
-        if (t0 + u * LPV < nm) L[t0 + u * LPV] = x[u];
+      if (fp & kPosBound)
+        for (int d = 0; d < 4; d++) fL[8 * pos + 4 + d] = 0.0;
     }
   }
   wsync_d();
-  const double *const Gm = GLOBAL ? pre : L;
-  const double *const Gh = Gm + mom_size(sym, ni);
   const int rounds = (ns + LPV - 1) / LPV;
   for (int t = lane; t < ns; t += LPV) {
-    if (t != lane) slot_load(a, se0 + t, r, mu0);
+    if (t != lane) slot_load<false>(a, se0 + t, r, mu0);
     slot_faces(A, r);
-    slot_fluxes<false>(A, ty, 0, r);
+    double S[3][3], q[3];
+    {
+      double H[3][3];
+      for (int i = 0; i < 3; i++)
+        for (int j = 0; j < 3; j++) H[i][j] = r.V[i] * r.Q[j];
+      if (r.posb >= 0) add_derived(H, r.Ab, r.ia2);
+      stress(H, r.mu, r.c2, r.c3, r.ivol, S);
+      const double qb = r.posb >= 0 ? dot3(r.Ab, r.Q) * r.ia2 : 0.0, kt = r.kv * r.th;
+      for (int d = 0; d < 3; d++) q[d] = kt * (r.Q[d] - r.Ab[d] * qb);
+    }
 #pragma unroll
     for (int e = 0; e < kSlotSrc; e++)
       if (e < r.ms) {
-        const int b = (r.code >> (8 * e)) & 0xFF, pos = b & kPosMask, side = b & kCodeRight ? 1 : 0;
-        for (int d = 0; d < 3; d++) fL[6 * pos + 3 * side + d] = r.g[e][d];
-        fh[2 * pos + side] = r.gh[e];
+        const int b = (r.code >> (8 * e)) & 0xFF;
+        double Ae[3];
+        load3(A, b & kPosMask, b & kCodeRight ? -1.0 : 1.0, Ae);
+        put4(fL + 8 * (b & kPosMask) + (b & kCodeRight ? 4 : 0), dot3(S[0], Ae), dot3(S[1], Ae), dot3(S[2], Ae),
+             dot3(q, Ae));
       }
   }
   wsync_d();
-  for (int q = lane; q < 3 * ni; q += LPV) {
-    const int l = q / 3, i = q - 3 * l;
-    double x = fL[6 * l + i] + fL[6 * l + 3 + i];
-    if (tag && (ty[l] & kTyV) == 2) x = a.p.bc_val_V[ty[l] >> kTyBc][i];
-    fv[q] = x;
-  }
-  for (int l = lane; l < ni; l += LPV) {
-    double x = fh[2 * l] + fh[2 * l + 1];
-    if (tag && (ty[l] >> kTyTShift & 3) == 2) x = a.p.bc_val_T[ty[l] >> kTyBc];
-    fhv[l] = x;
-  }
-  wsync_d();
-  double *const Vf = fL, *const Tf = fh;  // the face values take the one-sided fluxes' places
-  for (int q = lane; q < 3 * ni; q += LPV) {
-    const int l = q / 3, i = q - 3 * l;
-    double acc = 0.0;
-    for (int po = 0; po < ni; po++) {
-      const Blk b = block_at(sym, ni, l, po);
-      const double *x = Gm + b.base + b.si * i;
-      for (int j = 0; j < 3; j++) acc = acc + x[b.sj * j] * fv[3 * po + j];
+  for (int q = lane; q < 4 * ni; q += LPV) {
+    const int l = q >> 2, i = q & 3;
+    double f = fL[8 * l + i] + fL[8 * l + 4 + i];
+    if (tag) {
+      const int t = ty[l], ib = t >> kTyBc;
+      if (i < 3 ? (t & kTyV) == 2 : (t >> kTyTShift & 3) == 2) f = i < 3 ? a.p.bc_val_V[ib][i] : a.p.bc_val_T[ib];
     }
-    Vf[q] = acc;
-  }
-  for (int l = lane; l < ni; l += LPV) {
-    double acc = 0.0;
-    for (int po = 0; po < ni; po++) acc = acc + Gh[heat_at(sym, ni, l, po)] * fhv[po];
-    Tf[l] = acc;
+    fv[q] = f;
   }
   wsync_d();
+  if (GLOBAL) {
+    double *const vf = fL;
+    for (int q = lane; q < 3 * ni; q += LPV) {
+      const int l = q / 3, i = q - 3 * l;
+      double acc = 0.0;
+      for (int po = 0; po < ni; po++) {
+        const Blk b = block_at(sym, ni, l, po);
+        const double *y = pre + b.base + b.si * i;
+        for (int j = 0; j < 3; j++) acc = acc + y[b.sj * j] * fv[4 * po + j];
+      }
+      vf[4 * l + i] = acc;
+    }
+    const double *const ph = pre + mom_size(sym, ni);
+    for (int l = lane; l < ni; l += LPV) {
+      double acc = 0.0;
+      for (int po = 0; po < ni; po++) acc = acc + ph[heat_at(sym, ni, l, po)] * fv[4 * po + 3];
+      vf[4 * l + 3] = acc;
+    }
+  } else {
+    auto products = [&](int b, const double *y) {
+      int hi, lo;
+      if (sym) {
+        hi = (int)((sqrtf(8.0f * b + 1.0f) - 1.0f) * 0.5f);
+        lo = b - tri(hi);
+      } else {
+        hi = b / ni;
+        lo = b - hi * ni;
+      }
+      double f[4], g[4];
+      get4(fv + 4 * lo, f);
+      get4(fv + 4 * hi, g);
+      put4(fL + 4 * (hi * ni + lo), dot3(y, f), dot3(y + 3, f), dot3(y + 6, f), y[9] * f[3]);
+      if (sym && hi != lo)
+        put4(fL + 4 * (lo * ni + hi), y[0] * g[0] + y[3] * g[1] + y[6] * g[2], y[1] * g[0] + y[4] * g[1] + y[7] * g[2],
+             y[2] * g[0] + y[5] * g[1] + y[8] * g[2], y[9] * g[3]);
+    };
+#pragma unroll
+    for (int h = 0; h < kHold; h++)
+      if (lane + h * LPV < nb) products(lane + h * LPV, x[h]);
+    for (int b = lane + kHold * LPV; b < nb; b += LPV) {
+      double y[10];
+#pragma unroll
+      for (int k = 0; k < 10; k++) y[k] = pre[k * nb + b];
+      products(b, y);
+    }
+    wsync_d();
+    for (int q = lane; q < 4 * ni; q += LPV) {
+      const double *row = fL + 4 * ni * (q >> 2) + (q & 3);
+      double acc = 0.0;
+      for (int po = 0; po < ni; po++) acc = acc + row[4 * po];
+      fv[q] = acc;
+    }
+  }
+  wsync_d();
+  const double *const Vf = GLOBAL ? fL : fv;
   for (int t = lane; t < ns; t += LPV) {
     if (rounds > 1) {
-      slot_load(a, se0 + t, r, mu0);
+      slot_load<false>(a, se0 + t, r, mu0);
       slot_faces(A, r);
     }
     double H[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}}, h[3] = {0, 0, 0};
@@ -842,9 +917,10 @@ __global__ __launch_bounds__(256, 4) void k_visc_apply(DiffArgs a) {
     for (int e = 0; e < kSlotSrc; e++)
       if (e < r.ms) {
         const int be = (r.code >> (8 * e)) & 0xFF, pe = be & kPosMask;
-        double w[3], Ae[3];
-        for (int i = 0; i < 3; i++) w[i] = Vf[3 * pe + i] - r.V[i];
-        const double wt = Tf[pe] - r.th;
+        double w[4], Ae[3];
+        get4(Vf + 4 * pe, w);
+        for (int i = 0; i < 3; i++) w[i] = w[i] - r.V[i];
+        const double wt = w[3] - r.th;
         load3(A, pe, be & kCodeRight ? -1.0 : 1.0, Ae);
         for (int j = 0; j < 3; j++) {
           for (int i = 0; i < 3; i++) H[i][j] = H[i][j] + w[i] * Ae[j];
@@ -1137,8 +1213,7 @@ __global__ __launch_bounds__(256) void k_diff_expand(long C, const double *U, co
   for (int q = 0; q < 25; q++) diag[25 * c + q] = D[q];
 }
 
-hipError_t launch_lds(void (*fn)(DiffArgs), unsigned threads, int per, DiffArgs a, hipStream_t s) {
-  const size_t lds = sizeof(double) * per * a.lds_stride;
+hipError_t launch_lds(void (*fn)(DiffArgs), unsigned threads, int per, size_t lds, DiffArgs a, hipStream_t s) {
   if (lds > (64u << 10)) {
     hipError_t e = hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
@@ -1154,17 +1229,17 @@ hipError_t launch_visc(DiffArgs a, hipStream_t s) {
   constexpr bool FORM = MODE != kGlobal;
   a.lmat = FORM ? 10 * a.nim * a.nim : 0;
   a.lds_stride = lds_layout(a.lmat, a.nim, a.nfm, a.nsm, FORM).total;
-  return launch_lds(k_visc<LPV, MODE>, 64, 64 / LPV, a, s);
+  return launch_lds(k_visc<LPV, MODE>, 64, 64 / LPV, sizeof(double) * (64 / LPV) * a.lds_stride, a, s);
 }
 
 template <int LPV, bool GLOBAL>
 hipError_t launch_apply(DiffArgs a, hipStream_t s) {
-  if (GLOBAL) a.lmat = 0;
-  a.lds_stride = lds_layout(a.lmat, a.nim, a.nfm, a.nsm, false).total;
+  // doubles of LDS per wavefront: of the fullest one, or of the largest vertices
+  a.lds_stride = GLOBAL ? apply_lds<true>(a.nim, a.nfm) : a.lds_wave;
   // four wavefronts per workgroup where their LDS fits in 64 KB, else one
-  const bool four = sizeof(double) * (256 / LPV) * a.lds_stride <= (64u << 10);
-  const unsigned threads = four ? 256 : 64;
-  return launch_lds(k_visc_apply<LPV, GLOBAL>, threads, threads / LPV, a, s);
+  const unsigned threads = sizeof(double) * 4 * a.lds_stride <= (64u << 10) ? 256 : 64;
+  const size_t lds = sizeof(double) * (threads / 64) * a.lds_stride;
+  return launch_lds(k_visc_apply<LPV, GLOBAL>, threads, threads / LPV, lds, a, s);
 }
 
 }  // namespace
@@ -1222,6 +1297,8 @@ hipError_t launch_diff_terms(int cls, DiffArgs a, hipStream_t s) {
 hipError_t launch_diff_gather(DiffArgs a, hipStream_t s) {
   return a.mu_cell ? launch_gather<kDiffSlot>(a, 1, 1, s) : launch_gather<kDiffRow>(a, 1, 0, s);
 }
+
+int diff_apply_lds(int ni, int nf) { return apply_lds<false>(ni, nf); }
 
 hipError_t launch_diff_expand(long C, const double *U, const double *dblk, double cv, double *diag, hipStream_t s) {
   hipLaunchKernelGGL(k_diff_expand, dim3((unsigned)((C + 255) / 256)), dim3(256), 0, s, C, U, dblk, cv, diag);
