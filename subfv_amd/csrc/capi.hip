@@ -87,6 +87,7 @@ struct subfv_batch {
   // members with the generation each had when the tables were built
   std::vector<std::pair<subfv_ctx *, uint64_t>> members;
   int scheme = 0, total_g = 0, total_c = 0;
+  bool fold = false;  // the members' reductions are folded (kFoldBlocks)
   sfv::InstDesc *d_desc = nullptr;
   int *d_gtab = nullptr, *d_ctab = nullptr;
   size_t cap_desc = 0, cap_gtab = 0, cap_ctab = 0;
@@ -134,7 +135,7 @@ struct subfv_ctx {
   double *NGP = nullptr;  // [V][9] cached nodal-gradient pseudo-inverses (geometry only)
   double *W = nullptr;    // [C][6] primitives and sound speed of the state a residual works on
   bool ngp_ready = false;
-  double *blk = nullptr;
+  double *blk = nullptr, *oblk = nullptr;  // block minima: of vol / sum_lambda, of omega
   // viscous terms: the inverses of each vertex's nodal systems (once per mesh
   // with a constant viscosity, every residual with Sutherland's law)
   bool diff_on = false, diff_ready = false;
@@ -243,7 +244,7 @@ void free_mesh(subfv_ctx *c) {
   c->has_mesh = false;
   for (auto &u : c->U) u = nullptr;
   c->P = c->P2 = c->rhs = c->rhs2 = c->sl = c->sl2 = nullptr;
-  c->NG = c->VMM = c->G = c->vp = c->diag = c->blk = c->NGP = c->W = nullptr;
+  c->NG = c->VMM = c->G = c->vp = c->diag = c->blk = c->oblk = c->NGP = c->W = nullptr;
   c->ngp_ready = false;
   c->doff = nullptr;
   c->pre = c->PD = c->rdiff = c->dsivol = nullptr;
@@ -467,6 +468,7 @@ int upload_mesh(subfv_ctx *c) {
   if ((r = dalloc(c, &c->G, 15 * C))) return r;
   if ((r = dalloc(c, &c->vp, 3 * V))) return r;
   if ((r = dalloc(c, &c->blk, nblk(std::max(C, V), kCellThreads) + 64))) return r;
+  if ((r = dalloc(c, &c->oblk, nblk(C, kCellThreads)))) return r;
   HIPCHK(c, hipMemsetAsync(c->G, 0, sizeof(double) * 15 * C, c->stream));
   HIPCHK(c, hipMemsetAsync(c->NG, 0, sizeof(double) * 15 * V, c->stream));
   HIPCHK(c, hipMemsetAsync(c->vp, 0, sizeof(double) * 3 * V, c->stream));
@@ -531,11 +533,11 @@ int finish_mesh(subfv_ctx *c, int32_t boundary_2d) {
 // --------------------------------------------------------------- launches
 // c->W = the primitives and sound speeds of U, for the sweeps and gradients
 // of one residual
+int ensure_prim(subfv_ctx *c) { return c->W ? 0 : dalloc(c, &c->W, 6 * (size_t)c->dm.C); }
+
 int launch_prim(subfv_ctx *c, const double *U) {
-  if (!c->W) {
-    int r = dalloc(c, &c->W, 6 * (size_t)c->dm.C);
-    if (r) return r;
-  }
+  int r = ensure_prim(c);
+  if (r) return r;
   hipLaunchKernelGGL(k_prim, dim3(nblk(c->dm.C, 256)), dim3(256), 0, c->stream, (long)c->dm.C, U, c->W);
   HIPCHK(c, hipGetLastError());
   return 0;
@@ -579,7 +581,7 @@ int launch_flux(subfv_ctx *c, const double *U, const double *G, double *P, bool 
 }
 
 int launch_gather(subfv_ctx *c, const double *P, const double *P2, double *rhs, double *rhs2, double *sl,
-                  int fixed_dt) {
+                  int fixed_dt, bool fold = false) {
   GatherArgs g;
   g.m = c->dm;
   g.P = P;
@@ -595,8 +597,9 @@ int launch_gather(subfv_ctx *c, const double *P, const double *P2, double *rhs, 
   g.nblocks = nb;
   g.per_xcd = (nb + 7) / 8;
   hipLaunchKernelGGL(k_gather, dim3(8 * g.per_xcd), dim3(kCellThreads), 0, c->stream, g);
-  hipLaunchKernelGGL(k_finalize_dt, dim3(1), dim3(kCellThreads), 0, c->stream, (const double *)c->blk, nb, c->st,
-                     fixed_dt);
+  if (!fold)
+    hipLaunchKernelGGL(k_finalize_dt, dim3(1), dim3(kCellThreads), 0, c->stream, (const double *)c->blk, nb, c->st,
+                       fixed_dt);
   HIPCHK(c, hipGetLastError());
   return 0;
 }
@@ -637,18 +640,28 @@ int launch_grad(subfv_ctx *c, const double *U, int method, const double *W = nul
   return 0;
 }
 
+// fold: dt and omega are reduced inside the update and the correction
+// (kFoldBlocks), two launches instead of four with the gather's
 template <int DIAG>
-void launch_update_d(subfv_ctx *c, const UpdateArgs &u) {
-  dim3 g(nblk(c->dm.C, kCellThreads)), b(kCellThreads);
-  hipLaunchKernelGGL(k_update<DIAG>, g, b, 0, c->stream, u);
-  hipLaunchKernelGGL(k_finalize_omega, dim3(1), b, 0, c->stream, (const double *)c->blk, (int)g.x, c->st, u.advance_t);
+void launch_update_d(subfv_ctx *c, const UpdateArgs &u, bool fold) {
+  dim3 g(u.nblk), b(kCellThreads);
+  if (fold) {
+    hipLaunchKernelGGL((k_update<DIAG, true>), g, b, 0, c->stream, u);
+    hipLaunchKernelGGL(k_finish<DIAG>, g, b, 0, c->stream, u);
+    return;
+  }
+  hipLaunchKernelGGL((k_update<DIAG, false>), g, b, 0, c->stream, u);
+  hipLaunchKernelGGL(k_finalize_omega, dim3(1), b, 0, c->stream, (const double *)c->oblk, (int)g.x, c->st, u.advance_t);
   hipLaunchKernelGGL(k_update_fixup<DIAG>, g, b, 0, c->stream, u);
 }
+
+// a stage of a run folds its reductions where the mesh has few cell blocks
+bool folds(const subfv_ctx *c) { return nblk(c->dm.C, kCellThreads) <= (unsigned)kFoldBlocks; }
 
 // Ud: the state of the residual whose viscous terms enter (the stages of a run);
 // null: the diag array as it stands, its rhs already in rhs (the single update)
 int launch_update(subfv_ctx *c, const double *U, const double *U0, double *Uout, double a1, double a2, double w0,
-                  double w1, int flux_limit, int advance_t, const double *Ud = nullptr) {
+                  double w1, int flux_limit, int advance_t, const double *Ud = nullptr, int fixed_dt = 0) {
   UpdateArgs u;
   u.m = c->dm;
   u.U = U;
@@ -662,7 +675,11 @@ int launch_update(subfv_ctx *c, const double *U, const double *U0, double *Uout,
   u.Ud = Ud;
   u.dblk = c->dblk;
   u.cv = c->dparams.cv;
-  u.blk = c->blk;
+  u.W = Ud ? c->W : nullptr;  // a stage of a run: the next residual's primitives
+  u.dtblk = c->blk;
+  u.nblk = (int)nblk(c->dm.C, kCellThreads);
+  u.fixed_dt = fixed_dt;
+  u.blk = c->oblk;
   u.st = c->st;
   u.a1 = a1;
   u.a2 = a2;
@@ -671,12 +688,13 @@ int launch_update(subfv_ctx *c, const double *U, const double *U0, double *Uout,
   u.flux_limit = flux_limit;
   u.advance_t = advance_t;
   Prof pf(c, "update");
+  const bool fold = Ud && folds(c);
   if (c->diff_on && Ud)
-    launch_update_d<kDiagBlocks>(c, u);
+    launch_update_d<kDiagBlocks>(c, u, fold);
   else if (u.diag)
-    launch_update_d<kDiagFull>(c, u);
+    launch_update_d<kDiagFull>(c, u, fold);
   else
-    launch_update_d<kDiagNone>(c, u);
+    launch_update_d<kDiagNone>(c, u, fold);
   HIPCHK(c, hipGetLastError());
   return 0;
 }
@@ -1579,19 +1597,20 @@ int subfv_acoustic_run(subfv_ctx *c, double *sol, int32_t n_steps, double cfl, i
 }
 
 // One full residual evaluation on state U into rhs (and rhs2 in second
-// order), with dt from the first-order sum_lambda.
-static int residual(subfv_ctx *c, const double *U, int fixed_dt) {
+// order), with dt from the first-order sum_lambda.  first: U's primitives are not
+// yet in W (the update that wrote U leaves them there otherwise).
+static int residual(subfv_ctx *c, const double *U, int fixed_dt, bool first) {
   int r;
   if (c->diff_on && (r = launch_diffusion(c, U))) return r;
-  if ((r = launch_prim(c, U))) return r;
+  if (first && (r = launch_prim(c, U))) return r;
   if (c->cfg.second_order) {
     if ((r = launch_grad(c, U, c->cfg.method, c->W))) return r;
     if ((r = launch_flux(c, U, nullptr, c->P, false, c->W))) return r;
     if ((r = launch_flux(c, U, c->G, c->P2, false, c->W))) return r;
-    return launch_gather(c, c->P, c->P2, c->rhs, c->rhs2, c->sl, fixed_dt);
+    return launch_gather(c, c->P, c->P2, c->rhs, c->rhs2, c->sl, fixed_dt, folds(c));
   }
   if ((r = launch_flux(c, U, nullptr, c->P, false, c->W))) return r;
-  return launch_gather(c, c->P, nullptr, c->rhs, nullptr, c->sl, fixed_dt);
+  return launch_gather(c, c->P, nullptr, c->rhs, nullptr, c->sl, fixed_dt, folds(c));
 }
 
 int subfv_profile_enable(subfv_ctx *c, int32_t on) {
@@ -1760,11 +1779,11 @@ int subfv_run(subfv_ctx *c, int32_t n_steps, int32_t time_scheme, double *t, dou
   for (int it = 0; it < n_steps; it++) {
     int a = c->cur, b = (a + 1) % 3, q = (a + 2) % 3;
     if (time_scheme == 0) {
-      if ((r = residual(c, c->U[a], 0))) return r;
+      if ((r = residual(c, c->U[a], 0, it == 0))) return r;
       if (c->cfg.second_order) {
         // ns_main.F90:88-95: half step into U*, residual at U*, full step from U^n
         if ((r = launch_update(c, c->U[a], nullptr, c->U[b], 2.0, 1.0, 0.0, 1.0, fl, 0, c->U[a]))) return r;
-        if ((r = residual(c, c->U[b], 0))) return r;
+        if ((r = residual(c, c->U[b], 0, false))) return r;
         if ((r = launch_update(c, c->U[a], nullptr, c->U[q], 1.0, 1.0, 0.0, 1.0, fl, 1, c->U[b]))) return r;
         last = c->U[b];
         c->cur = q;
@@ -1775,12 +1794,12 @@ int subfv_run(subfv_ctx *c, int32_t n_steps, int32_t time_scheme, double *t, dou
       }
     } else {
       // SSP-RK3: U1 = L(Un) -> b; U2 = 3/4 Un + 1/4 L(U1) -> q; Un+1 = 1/3 Un + 2/3 L(U2) -> b
-      if ((r = residual(c, c->U[a], 0))) return r;
+      if ((r = residual(c, c->U[a], 0, it == 0))) return r;
       if ((r = launch_update(c, c->U[a], nullptr, c->U[b], 1.0, 1.0, 0.0, 1.0, fl, 0, c->U[a]))) return r;
-      if ((r = residual(c, c->U[b], 1))) return r;
-      if ((r = launch_update(c, c->U[b], c->U[a], c->U[q], 1.0, 1.0, 0.75, 0.25, fl, 0, c->U[b]))) return r;
-      if ((r = residual(c, c->U[q], 1))) return r;
-      if ((r = launch_update(c, c->U[q], c->U[a], c->U[b], 1.0, 1.0, 1.0 / 3.0, 2.0 / 3.0, fl, 2, c->U[q]))) return r;
+      if ((r = residual(c, c->U[b], 1, false))) return r;
+      if ((r = launch_update(c, c->U[b], c->U[a], c->U[q], 1.0, 1.0, 0.75, 0.25, fl, 0, c->U[b], 1))) return r;
+      if ((r = residual(c, c->U[q], 1, false))) return r;
+      if ((r = launch_update(c, c->U[q], c->U[a], c->U[b], 1.0, 1.0, 1.0 / 3.0, 2.0 / 3.0, fl, 2, c->U[q], 1))) return r;
       last = c->U[q];
       c->cur = b;
     }
@@ -2680,6 +2699,7 @@ void fill_desc(subfv_ctx *c, InstDesc &d) {
   d.fa.bc = c->bc;
   d.fa.U = nullptr;
   d.fa.G = nullptr;
+  d.fa.W = c->W;
   d.fa.P = c->P;
   d.fa.vp = nullptr;
   d.fa.err = c->derr;
@@ -2704,7 +2724,11 @@ void fill_desc(subfv_ctx *c, InstDesc &d) {
   d.ua.sl = c->sl;
   d.ua.diag = nullptr;
   d.ua.rdiff = nullptr;
-  d.ua.blk = c->blk;
+  d.ua.W = c->W;
+  d.ua.dtblk = c->blk;
+  d.ua.nblk = (int)nblk(c->dm.C, kCellThreads);
+  d.ua.fixed_dt = 0;
+  d.ua.blk = c->oblk;
   d.ua.st = c->st;
   d.ua.a1 = 1.0;
   d.ua.a2 = 1.0;
@@ -2725,9 +2749,16 @@ void launch_phase(subfv_batch *b, int n, int phase) {
                      (const InstDesc *)b->d_desc, (const int *)b->d_gtab, b->total_g, per_xcd, phase);
   hipLaunchKernelGGL(k_gather_multi, dim3(b->total_c), dim3(kCellThreads), 0, b->stream, (const InstDesc *)b->d_desc,
                      (const int *)b->d_ctab, b->total_c);
+  if (b->fold) {
+    hipLaunchKernelGGL(k_update_multi<true>, dim3(b->total_c), dim3(kCellThreads), 0, b->stream,
+                       (const InstDesc *)b->d_desc, (const int *)b->d_ctab, b->total_c, phase);
+    hipLaunchKernelGGL(k_finish_multi, dim3(b->total_c), dim3(kCellThreads), 0, b->stream,
+                       (const InstDesc *)b->d_desc, (const int *)b->d_ctab, b->total_c, phase);
+    return;
+  }
   hipLaunchKernelGGL(k_finalize_dt_multi, dim3(n), dim3(kCellThreads), 0, b->stream, (const InstDesc *)b->d_desc);
-  hipLaunchKernelGGL(k_update_multi, dim3(b->total_c), dim3(kCellThreads), 0, b->stream, (const InstDesc *)b->d_desc,
-                     (const int *)b->d_ctab, b->total_c, phase);
+  hipLaunchKernelGGL(k_update_multi<false>, dim3(b->total_c), dim3(kCellThreads), 0, b->stream,
+                     (const InstDesc *)b->d_desc, (const int *)b->d_ctab, b->total_c, phase);
   hipLaunchKernelGGL(k_finalize_omega_multi, dim3(n), dim3(kCellThreads), 0, b->stream, (const InstDesc *)b->d_desc);
   hipLaunchKernelGGL(k_update_fixup_multi, dim3(b->total_c), dim3(kCellThreads), 0, b->stream,
                      (const InstDesc *)b->d_desc, (const int *)b->d_ctab, b->total_c, phase);
@@ -2874,13 +2905,22 @@ int subfv_batch_run(subfv_batch *b, subfv_ctx **ctxs, int32_t n, int32_t n_steps
     BHIP(b, hipMemcpyAsync(b->d_ctab, ct.data(), ct.size() * sizeof(int), hipMemcpyHostToDevice, b->stream));
     b->total_g = (int)gt.size();
     b->total_c = (int)ct.size();
+    // dt and omega reduced inside the update and the correction, two launches
+    // less per step, unless a member has too many blocks for every one to reduce
+    b->fold = true;
+    for (int i = 0; i < n; i++) b->fold = b->fold && folds(ctxs[i]);
     batch_drop_graph(b);
   }
   int r;
   if ((r = grow(b, &b->d_desc, &b->cap_desc, (size_t)n))) return r;
+  for (int i = 0; i < n; i++)
+    if ((r = ensure_prim(ctxs[i]))) return bfail(b, r, ctxs[i]->err);
   std::vector<InstDesc> hd(n);
   for (int i = 0; i < n; i++) fill_desc(ctxs[i], hd[i]);
   BHIP(b, hipMemcpyAsync(b->d_desc, hd.data(), n * sizeof(InstDesc), hipMemcpyHostToDevice, b->stream));
+  if (n_steps > 0)
+    hipLaunchKernelGGL(k_prim_multi, dim3(b->total_c), dim3(kCellThreads), 0, b->stream, (const InstDesc *)b->d_desc,
+                       (const int *)b->d_ctab, b->total_c);
   int s = 0;
   if (use_graph == 2 && n_steps > 0) {
     if ((r = launch_persistent_any(b, n, n_steps))) return r;

@@ -62,13 +62,33 @@ __global__ __launch_bounds__(kCellThreads) void k_finalize_dt_multi(const InstDe
   finalize_dt(D.ga.blk, D.ncblk, D.ga.st, 0);
 }
 
+template <bool FOLD>
 __global__ __launch_bounds__(kCellThreads) void k_update_multi(const InstDesc *d, const int *ctab, int total,
                                                                int phase) {
   if ((int)blockIdx.x >= total) return;
   const int e = ctab[blockIdx.x];
   const InstDesc &D = *(const InstDesc *)((const CInstDesc *)d + (e >> kTabShift));
   if ((e & kTabMask) >= D.ncblk) return;
-  update_block<false>(D.ua, D.U[(D.cur0 + phase) % 3], D.U[(D.cur0 + phase + 1) % 3], e & kTabMask);
+  update_block<kDiagNone, FOLD>(D.ua, D.U[(D.cur0 + phase) % 3], D.U[(D.cur0 + phase + 1) % 3], e & kTabMask);
+}
+
+// the primitives of every instance's current state
+__global__ __launch_bounds__(kCellThreads) void k_prim_multi(const InstDesc *d, const int *ctab, int total) {
+  if ((int)blockIdx.x >= total) return;
+  const int e = ctab[blockIdx.x];
+  const InstDesc &D = *(const InstDesc *)((const CInstDesc *)d + (e >> kTabShift));
+  if ((e & kTabMask) >= D.ncblk) return;
+  prim_block(D.ua.m.C, D.U[D.cur0 % 3], D.ua.W, e & kTabMask);
+}
+
+// k_finalize_omega_multi and k_update_fixup_multi in one (finish_block)
+__global__ __launch_bounds__(kCellThreads) void k_finish_multi(const InstDesc *d, const int *ctab, int total,
+                                                               int phase) {
+  if ((int)blockIdx.x >= total) return;
+  const int e = ctab[blockIdx.x];
+  const InstDesc &D = *(const InstDesc *)((const CInstDesc *)d + (e >> kTabShift));
+  if ((e & kTabMask) >= D.ncblk) return;
+  finish_block<kDiagNone>(D.ua, D.U[(D.cur0 + phase) % 3], D.U[(D.cur0 + phase + 1) % 3], e & kTabMask);
 }
 
 __global__ __launch_bounds__(kCellThreads) void k_finalize_omega_multi(const InstDesc *d) {
@@ -82,7 +102,7 @@ __global__ __launch_bounds__(kCellThreads) void k_update_fixup_multi(const InstD
   const int e = ctab[blockIdx.x];
   const InstDesc &D = *(const InstDesc *)((const CInstDesc *)d + (e >> kTabShift));
   if ((e & kTabMask) >= D.ncblk) return;
-  update_fixup_block<false>(D.ua, D.U[(D.cur0 + phase) % 3], D.U[(D.cur0 + phase + 1) % 3], e & kTabMask);
+  update_fixup_block<kDiagNone>(D.ua, D.U[(D.cur0 + phase) % 3], D.U[(D.cur0 + phase + 1) % 3], e & kTabMask);
 }
 
 // ------------------------------------------------------- persistent form
@@ -162,7 +182,7 @@ __global__ __launch_bounds__(kGrpThreads, 3) void k_batch_persistent(PersistArgs
       const int e = a.ctab[k], i = e >> kTabShift;
       const InstDesc &D = *(const InstDesc *)((const CInstDesc *)a.d + i);
       if ((e & kTabMask) >= D.ncblk) continue;
-      update_block<false>(D.ua, D.U[(D.cur0 + phase) % 3], D.U[(D.cur0 + phase + 1) % 3], e & kTabMask);
+      update_block<kDiagNone, false>(D.ua, D.U[(D.cur0 + phase) % 3], D.U[(D.cur0 + phase + 1) % 3], e & kTabMask);
       if (last_arrival(dn + a.n_inst + i, D.ncblk, &s_flag)) finalize_omega(D.ua.blk, D.ncblk, D.ua.st, 1);
       __syncthreads();
     }
@@ -171,7 +191,7 @@ __global__ __launch_bounds__(kGrpThreads, 3) void k_batch_persistent(PersistArgs
       const int e = a.ctab[k];
       const InstDesc &D = *(const InstDesc *)((const CInstDesc *)a.d + (e >> kTabShift));
       if ((e & kTabMask) >= D.ncblk) continue;
-      update_fixup_block<false>(D.ua, D.U[(D.cur0 + phase) % 3], D.U[(D.cur0 + phase + 1) % 3], e & kTabMask);
+      update_fixup_block<kDiagNone>(D.ua, D.U[(D.cur0 + phase) % 3], D.U[(D.cur0 + phase + 1) % 3], e & kTabMask);
       __syncthreads();
     }
     grid.sync();

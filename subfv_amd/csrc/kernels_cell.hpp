@@ -23,6 +23,7 @@ struct StepState {
   int lts;             // local_time_step
   unsigned int ticket; // last-block-done counter
   int steps;           // completed steps
+  int frozen;          // done or err when the last update began
 };
 
 constexpr int kCellThreads = 256;
@@ -76,11 +77,8 @@ __global__ __launch_bounds__(kCellThreads) void k_finalize_dt(const double *blk,
   finalize_dt(blk, nblk, st, fixed_dt);
 }
 
-// omega checks and time advance of add_timedisc_and_solve (:595-608)
-SFV_DEV void finalize_omega(const double *blk, int nblk, StepState *st, int advance_t) {
-  double om = reduce_min_one_block(blk, nblk);
-  if (threadIdx.x != 0) return;
-  if (st->done || st->err) return;
+// omega checks and time advance of add_timedisc_and_solve (:595-608), one thread
+SFV_DEV void advance_state(StepState *st, double om, int advance_t) {
   double omega = dmin(1.0, om);
   st->omega_min = om;
   st->omega = omega;
@@ -98,6 +96,15 @@ SFV_DEV void finalize_omega(const double *blk, int nblk, StepState *st, int adva
     st->steps += 1;
     if (!st->lts && st->t >= st->tmax) st->done = 1;
   }
+}
+SFV_DEV void finalize_omega(const double *blk, int nblk, StepState *st, int advance_t) {
+  double om = reduce_min_one_block(blk, nblk);
+  if (threadIdx.x != 0) return;
+  if (st->done || st->err) {
+    st->fixup = 0;  // a frozen state takes no correction
+    return;
+  }
+  advance_state(st, om, advance_t);
 }
 __global__ __launch_bounds__(kCellThreads) void k_finalize_omega(const double *blk, int nblk, StepState *st,
                                                                  int advance_t) {
@@ -182,7 +189,11 @@ struct UpdateArgs {
   const double *Ud, *dblk;  // the residual's state and the cells' viscous blocks (kDiagBlocks)
   double cv;
   const double *rdiff;// [C][4] viscous rhs of components 2..5 (added after flux limiting), or null
-  double *blk;
+  double *W;          // [C][6] primitives and sound speed of Uout (as k_prim), or null
+  const double *dtblk;// the gather's block minima, nblk of them (the folded forms)
+  double *blk;        // block minima of omega
+  int nblk;           // cell blocks
+  int fixed_dt;       // keep st->dt (the folded forms; SSP-RK3 stages 2 and 3)
   StepState *st;
   double a1, a2, w0, w1;
   int flux_limit;     // second order: flux_limiting before the update
@@ -196,10 +207,13 @@ enum { kDiagNone = 0, kDiagFull = 1, kDiagBlocks = 2 };
 // flux_limiting (ns_euler_recon_module.F90:586-593) + the per-cell part of
 // add_timedisc_and_solve (ns_euler_module.F90:565-580).  Returns the cell's
 // omega; u and delta receive the state and the increment.
+struct StepDt {
+  double dt, dt_fl;
+  int lts;
+};
 template <int DIAG>
-SFV_DEV double stage_cell(const UpdateArgs &a, const double *U, long c, double *u, double *delta) {
+SFV_DEV double stage_cell(const UpdateArgs &a, const StepDt &st, const double *U, long c, double *u, double *delta) {
   const long C = a.m.C;
-  const StepState *st = a.st;
   double r[5];
   for (int k = 0; k < 5; k++) {
     u[k] = U[5 * c + k];
@@ -209,7 +223,7 @@ SFV_DEV double stage_cell(const UpdateArgs &a, const double *U, long c, double *
   const double lam = a.sl[c];
   if (a.flux_limit) {
     double r2[5], x[5], y[5];
-    double cf = vol / st->dt_fl + lam;
+    double cf = vol / st.dt_fl + lam;
     for (int k = 0; k < 5; k++) {
       r2[k] = a.rhs2[k * C + c];
       x[k] = u[k] + r[k] / cf;
@@ -220,7 +234,7 @@ SFV_DEV double stage_cell(const UpdateArgs &a, const double *U, long c, double *
   }
   if (DIAG && a.rdiff)  // the diffusion block follows flux limiting (ns_main.F90:170-175)
     for (int k = 1; k < 5; k++) r[k] = r[k] + a.rdiff[4 * c + k - 1];
-  double cc = a.a1 * (vol / st->dt + (st->lts ? lam : 0.0));
+  double cc = a.a1 * (vol / st.dt + (st.lts ? lam : 0.0));
   double nw[5];
   if (DIAG) {
     double D[25];
@@ -246,34 +260,68 @@ SFV_DEV double stage_cell(const UpdateArgs &a, const double *U, long c, double *
 
 SFV_DEV void store_stage(const UpdateArgs &a, double *Uout, long c, const double *u, const double *delta,
                          double omega) {
+  double y[5];
   for (int k = 0; k < 5; k++) {
     double x = u[k] + a.a2 * omega * delta[k];
     if (a.U0) x = a.w0 * a.U0[5 * c + k] + a.w1 * x;
     Uout[5 * c + k] = x;
+    y[k] = x;
   }
+  if (a.W) cell_prim(y, a.W + 6 * c);
 }
 
-template <int DIAG>
+// The step's dt.  FOLD: every block reduces the gather's minima itself, as
+// finalize_dt does, and the first writes the state; otherwise finalize_dt ran
+// before.  One reduction per block is nothing up to kFoldBlocks blocks, and a
+// launch of one block (4 us) less; beyond, the blocks' reads would add up.
+constexpr int kFoldBlocks = 1024;
+template <bool FOLD>
+SFV_DEV StepDt step_dt(const UpdateArgs &a, long bidx) {
+  StepState *st = a.st;
+  StepDt r = {st->dt, st->dt_fl, st->lts};
+  if (FOLD) {
+    const double d = dmin(1e10, reduce_min_one_block(a.dtblk, a.nblk));
+    r.dt_fl = st->cfl * d;
+    if (!a.fixed_dt) {
+      r.dt = st->cfl * d;
+      if (!r.lts) r.dt = dmin(st->tmax - st->t + 1e-12, r.dt);
+    }
+    if (bidx == 0 && threadIdx.x == 0) {
+      st->dtmin = d;
+      st->dt_fl = r.dt_fl;
+      if (!a.fixed_dt) st->dt = r.dt;
+    }
+  }
+  return r;
+}
+
+template <int DIAG, bool FOLD>
 SFV_DEV void update_block(const UpdateArgs &a, const double *U, double *Uout, long bidx) {
   long c = bidx * kCellThreads + threadIdx.x;
   StepState *st = a.st;
-  if (st->done || st->err) {  // uniform over the grid: the state is frozen
-    if (c < a.m.C)
-      for (int k = 0; k < 5; k++) Uout[5 * c + k] = U[5 * c + k];
+  const int frozen = st->done || st->err;  // uniform over the grid: the state is frozen
+  const StepDt sd = step_dt<FOLD>(a, bidx);
+  if (FOLD && bidx == 0 && threadIdx.x == 0) st->frozen = frozen;
+  if (frozen) {
+    if (c < a.m.C) {
+      double u[5];
+      for (int k = 0; k < 5; k++) Uout[5 * c + k] = u[k] = U[5 * c + k];
+      if (a.W) cell_prim(u, a.W + 6 * c);
+    }
     return;
   }
   double om_c = 1.0;
   if (c < a.m.C) {
     double u[5], d[5];
-    om_c = stage_cell<DIAG>(a, U, c, u, d);
+    om_c = stage_cell<DIAG>(a, sd, U, c, u, d);
     store_stage(a, Uout, c, u, d, 1.0);
   }
   block_min_store(om_c, a.blk, (int)bidx);
 }
 
-template <int DIAG>
+template <int DIAG, bool FOLD>
 __global__ __launch_bounds__(kCellThreads) void k_update(UpdateArgs a) {
-  update_block<DIAG>(a, a.U, a.Uout, blockIdx.x);
+  update_block<DIAG, FOLD>(a, a.U, a.Uout, blockIdx.x);
 }
 
 // Correction when the global omega came out below one: redo the cell with
@@ -285,13 +333,36 @@ SFV_DEV void update_fixup_block(const UpdateArgs &a, const double *U, double *Uo
   if (!st->fixup || st->err) return;
   if (c >= a.m.C) return;
   double u[5], d[5];
-  stage_cell<DIAG>(a, U, c, u, d);
+  stage_cell<DIAG>(a, {st->dt, st->dt_fl, st->lts}, U, c, u, d);
   store_stage(a, Uout, c, u, d, st->omega);
 }
 
 template <int DIAG>
 __global__ __launch_bounds__(kCellThreads) void k_update_fixup(UpdateArgs a) {
   update_fixup_block<DIAG>(a, a.U, a.Uout, blockIdx.x);
+}
+
+// finalize_omega and the correction in one: every block reduces the minima; the
+// first advances the state, reading what the update left in frozen and not the
+// done and err that it writes.
+template <int DIAG>
+SFV_DEV void finish_block(const UpdateArgs &a, const double *U, double *Uout, long bidx) {
+  StepState *st = a.st;
+  if (st->frozen) return;  // uniform over the grid
+  const double om = reduce_min_one_block(a.blk, a.nblk);
+  const double omega = dmin(1.0, om);
+  const bool bad = omega <= 1e-6;
+  if (bidx == 0 && threadIdx.x == 0) advance_state(st, om, a.advance_t);
+  if (bad || !(omega < 1.0)) return;
+  const long c = bidx * kCellThreads + threadIdx.x;
+  if (c >= a.m.C) return;
+  double u[5], d[5];
+  stage_cell<DIAG>(a, {st->dt, st->dt_fl, st->lts}, U, c, u, d);
+  store_stage(a, Uout, c, u, d, omega);
+}
+template <int DIAG>
+__global__ __launch_bounds__(kCellThreads) void k_finish(UpdateArgs a) {
+  finish_block<DIAG>(a, a.U, a.Uout, blockIdx.x);
 }
 
 // ---------------------------------------------------------------- gradients

@@ -461,16 +461,24 @@ SFV_DEV void node_flux_group(const FluxArgs &a, const double *__restrict__ U, in
   }
 }
 
-// W[6 c + k] = conserv_to_primit(U_c)(k), W[6 c + 5] = sound_speed_w of it:
-// the cell values every sub-face of the sweeps would otherwise recompute
-static __global__ __launch_bounds__(256) void k_prim(long C, const double *__restrict__ U, double *__restrict__ W) {
-  const long c = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= C) return;
-  double u[5], w[5];
-  for (int k = 0; k < 5; k++) u[k] = U[5 * c + k];
+// w[0..4] = conserv_to_primit(u), w[5] = its sound_speed_w: the cell values every
+// sub-face of the sweeps would otherwise recompute.  A stage's update leaves those
+// of the state that it writes; k_prim forms them for the first.
+SFV_DEV void cell_prim(const double *u, double *W) {
+  double w[5];
   to_prim(u, w);
-  for (int k = 0; k < 5; k++) W[6 * c + k] = w[k];
-  W[6 * c + 5] = sound_speed(w);
+  for (int k = 0; k < 5; k++) W[k] = w[k];
+  W[5] = sound_speed(w);
+}
+SFV_DEV void prim_block(long C, const double *U, double *W, long bidx) {
+  const long c = bidx * 256 + threadIdx.x;
+  if (c >= C) return;
+  double u[5];
+  for (int k = 0; k < 5; k++) u[k] = U[5 * c + k];
+  cell_prim(u, W + 6 * c);
+}
+static __global__ __launch_bounds__(256) void k_prim(long C, const double *__restrict__ U, double *__restrict__ W) {
+  prim_block(C, U, W, blockIdx.x);
 }
 
 template <int SCHEME>

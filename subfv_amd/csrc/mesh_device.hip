@@ -169,7 +169,7 @@ __global__ void k_bfs_assign(int n, const int *sorted, int iloc, int *otn, int *
 }
 
 // Whole levels by one workgroup, without host reads or sorts: while the
-// frontier has at most kBfsCap vertices.  Eight lanes take a frontier vertex, an
+// frontier has at most cap <= kBfsCap vertices.  Eight lanes take a frontier vertex, an
 // element each.  (1) an unvisited vertex keeps the smallest key (place of the
 // frontier vertex, its element, the corner) that meets it, the reference's scan
 // order; (2) each frontier vertex counts the vertices whose kept key is its own;
@@ -186,7 +186,7 @@ constexpr int kBfsCap = 2048;
 constexpr int kBfsThreads = 1024;
 __global__ __launch_bounds__(kBfsThreads) void k_bfs_levels(int nv, const int *v_eoff, const int *v_elem,
                                                             const int *e_voff, const int *e_vert, int *otn, int *nto,
-                                                            unsigned long long *prio, int *pos) {
+                                                            unsigned long long *prio, int *pos, int cap) {
   __shared__ int base[kBfsCap];
   __shared__ int wsum[kBfsThreads / 64];
   __shared__ int s_first;
@@ -248,7 +248,7 @@ __global__ __launch_bounds__(kBfsThreads) void k_bfs_levels(int nv, const int *v
   int iloc = pos[0], istart = pos[1], iend = pos[2], cursor = pos[3];
   while (iloc < nv) {
     const int nfront = iend - istart + 1;
-    if (nfront > kBfsCap) break;
+    if (nfront > cap) break;
     for (int i = tid >> 3; i < nfront; i += kPer) {
       const int v = nto[istart + i], b = v_eoff[v], e = v_eoff[v + 1];
       for (int q = b + sub; q < e; q += 8) {
@@ -781,13 +781,16 @@ std::string build_device_mesh(HostMesh &m, int nv, const double *coord, int ne, 
     c.chk(hipMemcpyAsync(nto.p, &zero, sizeof(int), hipMemcpyHostToDevice, c.s));
     c.chk(hipStreamSynchronize(c.s));
   }
+  // a frontier of about 40,000 corners to look at (1,100 vertices of a prism mesh,
+  // 400 of a tetrahedral one) takes one workgroup as long as the launches take
+  const int cap = (int)std::min<double>(kBfsCap, 4e4 / ((double)nq / nv * nq / ne));
   int hpos[4] = {1, 0, 0, 0};  // iloc, istart, iend, cursor of k_bfs_levels
   while (hpos[0] < nv && !c.err) {
     int &iloc = hpos[0], &istart = hpos[1], &iend = hpos[2];
-    if (iend - istart + 1 <= kBfsCap) {
+    if (iend - istart + 1 <= cap) {
       c.chk(hipMemcpyAsync(pos.p, hpos, sizeof(hpos), hipMemcpyHostToDevice, c.s));
       hipLaunchKernelGGL(k_bfs_levels, dim3(1), dim3(kBfsThreads), 0, c.s, nv, (const int *)v_eoff, (const int *)v_elem,
-                         (const int *)d_evoff, (const int *)d_evert, otn.p, nto.p, prio64.p, pos.p);
+                         (const int *)d_evoff, (const int *)d_evert, otn.p, nto.p, prio64.p, pos.p, cap);
       c.chk(hipGetLastError());
       c.chk(hipMemcpyAsync(hpos, pos.p, sizeof(hpos), hipMemcpyDeviceToHost, c.s));
       c.chk(hipStreamSynchronize(c.s));
