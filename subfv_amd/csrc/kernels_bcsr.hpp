@@ -404,6 +404,9 @@ constexpr int kDchBeta0 = 2 * (kGsMax + 2), kDchCoef = kDchBeta0 + 1, kDchSize =
 constexpr int kDcCoefThreads = 1024, kDcRuns = 16, kDcPer = kGsBlocks / kDcRuns;
 static_assert(kGsBlocks % kDcRuns == 0, "partials split evenly into runs");
 
+// where block b's partial of a column lies: run b / kDcPer, entry b % kDcPer
+SFV_DEV int dc_part(int b) { return b % kDcPer * kDcRuns + b / kDcPer; }
+
 // sum over the 2^L lanes of each aligned group (xor butterfly, fixed order)
 template <int L>
 SFV_DEV double group_sum(double v) {
@@ -426,14 +429,16 @@ __global__ __launch_bounds__(kDcCoefThreads) void k_dc_coef(int s, const double 
     if (k < s - 1) hs[i][k] = i <= k + 1 ? H[i + (long)ldh * k] : 0.0;
   }
   // kDcRuns threads per partial column, each a fixed run of kDcPer blocks
-  // (loaded together, then added in order), then the runs in order
+  // (loaded together, then added in order), then the runs in order.  The runs
+  // are interleaved in memory (dc_part), so the kDcRuns threads of a column
+  // read one 128-byte line per load instead of a line each.
   for (int c0 = 0; c0 < ncol; c0 += kDcCoefThreads / kDcRuns) {
     const int c = c0 + (int)(threadIdx.x / kDcRuns), r = threadIdx.x % kDcRuns;
     if (c < ncol) {
-      const double *pp = part + (long)c * kGsBlocks + r * kDcPer;
+      const double *pp = part + (long)c * kGsBlocks + r;
       double v[kDcPer];
 #pragma unroll
-      for (int b = 0; b < kDcPer; b++) v[b] = pp[b];
+      for (int b = 0; b < kDcPer; b++) v[b] = pp[b * kDcRuns];
       double t = 0.0;
 #pragma unroll
       for (int b = 0; b < kDcPer; b++) t = t + v[b];
@@ -515,7 +520,7 @@ template <> struct Pair<double> { using T = double2; };
 template <> struct Pair<float> { using T = float2; };
 
 // The step's dot pass: per-block partials of a (columns 0..s-1), b
-// (s..2s-1), c (2s) and d (2s+1) into part[q * gridDim.x + blockIdx.x].  Each
+// (s..2s-1), c (2s) and d (2s+1) into part[q * kGsBlocks + dc_part(block)].  Each
 // thread takes two consecutive elements per iteration (ldv even); an odd n's
 // last element goes to thread 0.
 template <int KM, typename VT>
@@ -569,7 +574,7 @@ __global__ __launch_bounds__(kVecThreads) void k_dc_dot(long n, int s, const VT 
     const int src = t < s ? t : (t < 2 * s ? KM + (t - s) : 2 * KM + (t - 2 * s));
     double v = sh[0][src];
     for (int q = 1; q < kVecThreads / 64; q++) v = v + sh[q][src];
-    part[(long)t * gridDim.x + blockIdx.x] = v;
+    part[(long)t * kGsBlocks + dc_part(blockIdx.x)] = v;  // gridDim.x = kGsBlocks
   }
 }
 
