@@ -278,12 +278,14 @@ struct Prof {
   }
 };
 
-int check_err(subfv_ctx *c) {
+// the error bits of everything queued so far; out: the step state read with them
+int check_err(subfv_ctx *c, StepState *out = nullptr) {
   int e = 0;
   HIPCHK(c, hipMemcpyAsync(&e, c->derr, sizeof(int), hipMemcpyDeviceToHost, c->stream));
   StepState hs;
   HIPCHK(c, hipMemcpyAsync(&hs, c->st, sizeof(StepState), hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
+  if (out) *out = hs;
   int bits = e | hs.err;
   if (bits & kErrNegStarDensity) return fail(c, SUBFV_E_NEG_STAR, "Negative specific volume MPCC !");
   if (bits & kErrBadOmega) return fail(c, SUBFV_E_BAD_OMEGA, "BAD OMEGA " + std::to_string(hs.omega_min));
@@ -1377,13 +1379,18 @@ int64_t subfv_put_f64(subfv_ctx *c, const char *name, const double *in, int64_t 
   return -1;
 }
 
-int subfv_compute_euler_flux(subfv_ctx *c, int32_t second_order, int32_t want_vp) {
-  if (!c || !c->has_mesh) return fail(c, SUBFV_E_INVALID, "no mesh");
+// the launches of compute_euler_flux
+static int queue_euler_flux(subfv_ctx *c, int32_t second_order, int32_t want_vp) {
   const double *U = c->U[c->cur];
   double *P = second_order ? c->P2 : c->P;
   int r = launch_flux(c, U, second_order ? c->G : nullptr, P, want_vp != 0);
   if (r) return r;
-  r = launch_gather(c, P, nullptr, second_order ? c->rhs2 : c->rhs, nullptr, second_order ? c->sl2 : c->sl, 1);
+  return launch_gather(c, P, nullptr, second_order ? c->rhs2 : c->rhs, nullptr, second_order ? c->sl2 : c->sl, 1);
+}
+
+int subfv_compute_euler_flux(subfv_ctx *c, int32_t second_order, int32_t want_vp) {
+  if (!c || !c->has_mesh) return fail(c, SUBFV_E_INVALID, "no mesh");
+  int r = queue_euler_flux(c, second_order, want_vp);
   if (r) return r;
   return check_err(c);
 }
@@ -1397,23 +1404,24 @@ int subfv_compute_cell_grad(subfv_ctx *c, int32_t method) {
   return 0;
 }
 
+// the launches of flux_limiting: dt from the first-order sum_lambda with the
+// given cfl, the state's own cfl afterwards
+static int queue_flux_limiting(subfv_ctx *c, double cfl) {
+  const DevMesh &d = c->dm;
+  const unsigned nb = nblk(d.C, kCellThreads);
+  hipLaunchKernelGGL(k_dt_from_sl, dim3(nb), dim3(kCellThreads), 0, c->stream, d, c->sl, c->blk);
+  hipLaunchKernelGGL(k_finalize_dt_cfl, dim3(1), dim3(kCellThreads), 0, c->stream, (const double *)c->blk, (int)nb,
+                     c->st, cfl, c->cfg.cfl);
+  hipLaunchKernelGGL(k_flux_limiting, dim3(nb), dim3(kCellThreads), 0, c->stream, d, c->U[c->cur], c->rhs, c->rhs2,
+                     c->sl, c->st);
+  HIPCHK(c, hipGetLastError());
+  return 0;
+}
+
 int subfv_flux_limiting(subfv_ctx *c, double cfl) {
   if (!c || !c->has_mesh) return fail(c, SUBFV_E_INVALID, "no mesh");
-  StepState hs;
-  int r = sync_state_scalars(c, &hs);
+  int r = queue_flux_limiting(c, cfl);
   if (r) return r;
-  hs.cfl = cfl;
-  HIPCHK(c, hipMemcpyAsync(c->st, &hs, sizeof(StepState), hipMemcpyHostToDevice, c->stream));
-  const DevMesh &d = c->dm;
-  hipLaunchKernelGGL(k_dt_from_sl, dim3(nblk(d.C, kCellThreads)), dim3(kCellThreads), 0, c->stream, d, c->sl,
-                     c->blk);
-  hipLaunchKernelGGL(k_finalize_dt, dim3(1), dim3(kCellThreads), 0, c->stream, (const double *)c->blk,
-                     (int)nblk(d.C, kCellThreads), c->st, 0);
-  hipLaunchKernelGGL(k_flux_limiting, dim3(nblk(d.C, kCellThreads)), dim3(kCellThreads), 0, c->stream, d,
-                     c->U[c->cur], c->rhs, c->rhs2, c->sl, c->st);
-  HIPCHK(c, hipGetLastError());
-  hs.cfl = c->cfg.cfl;
-  HIPCHK(c, hipMemcpyAsync(&c->st->cfl, &hs.cfl, sizeof(double), hipMemcpyHostToDevice, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   return 0;
 }
@@ -1447,18 +1455,19 @@ int subfv_add_timedisc_and_solve(subfv_ctx *c, double a1, double a2, double cfl,
   return 0;
 }
 
+// The whole residual is queued and its error bits read once at the end (a read
+// and its synchronisation after every part took longer than a small mesh's
+// kernels); like the parts, it does not change the state.
 int subfv_compute_rhs_ns(subfv_ctx *c) {
   if (!c || !c->has_mesh) return fail(c, SUBFV_E_INVALID, "no mesh");
-  int r = subfv_compute_euler_flux(c, 0, 1);
+  int r = queue_euler_flux(c, 0, 1);
   if (r) return r;
   if (c->cfg.second_order) {
-    r = subfv_compute_cell_grad(c, c->cfg.method);
-    if (r) return r;
-    r = subfv_compute_euler_flux(c, 1, 1);
-    if (r) return r;
-    r = subfv_flux_limiting(c, c->cfg.cfl);
-    if (r) return r;
+    if ((r = launch_grad(c, c->U[c->cur], c->cfg.method))) return r;
+    if ((r = queue_euler_flux(c, 1, 1))) return r;
+    if ((r = queue_flux_limiting(c, c->cfg.cfl))) return r;
   }
+  if ((r = check_err(c))) return r;
   if (c->diff_on) {
     // the diffusion block (ns_main.F90:170-175): rhs += viscous terms, diag = their block
     r = launch_diffusion(c, c->U[c->cur]);
@@ -1805,13 +1814,13 @@ int subfv_run(subfv_ctx *c, int32_t n_steps, int32_t time_scheme, double *t, dou
     }
   }
   if (last && c->diff_on && (r = expand_diag(c, last))) return r;
-  StepState hs;
-  r = sync_state_scalars(c, &hs);
-  if (r) return r;
+  StepState hs{};
+  hs.t = c->host_t;
+  r = check_err(c, &hs);
   if (t) *t = hs.t;
   if (dt) *dt = (time_scheme == 0) ? hs.dt_adv : hs.dt;
   c->host_t = hs.t;
-  return check_err(c);
+  return r;
 }
 
 }  // extern "C"

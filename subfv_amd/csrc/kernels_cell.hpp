@@ -77,6 +77,14 @@ __global__ __launch_bounds__(kCellThreads) void k_finalize_dt(const double *blk,
   finalize_dt(blk, nblk, st, fixed_dt);
 }
 
+// the same with the given cfl, which the state keeps only while it is used
+__global__ __launch_bounds__(kCellThreads) void k_finalize_dt_cfl(const double *blk, int nblk, StepState *st,
+                                                                  double cfl, double cfl_after) {
+  if (threadIdx.x == 0) st->cfl = cfl;
+  finalize_dt(blk, nblk, st, 0);  // thread 0 reads the state after its own write
+  if (threadIdx.x == 0) st->cfl = cfl_after;
+}
+
 // omega checks and time advance of add_timedisc_and_solve (:595-608), one thread
 SFV_DEV void advance_state(StepState *st, double om, int advance_t) {
   double omega = dmin(1.0, om);
