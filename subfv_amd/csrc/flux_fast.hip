@@ -12,7 +12,7 @@
 namespace sfv {
 
 template <int SCHEME>
-__global__ __launch_bounds__(kGrpThreads, 3) void k_node_flux_fast(FluxArgs a) {
+__global__ __launch_bounds__(kGrpThreads, 4) void k_node_flux_fast(FluxArgs a) {
   __shared__ FluxLds L;
   const int lb = xcd_block(a.per_xcd);
   if (lb >= a.nblocks) return;  // uniform over the workgroup

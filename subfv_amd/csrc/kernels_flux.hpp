@@ -16,12 +16,14 @@
 // whole wavefronts' work, and the wall faces of one-layer meshes, whose lambdas
 // stand still from the second iteration on, skip its divisions and rows
 // together.  A group whose lambdas all stand leaves the iterations.  Divisions
-// that share a divisor share its reciprocal (quot).  What bounds the sweep is
-// latency between the barriers (VALU issue 47 %, LDS 25 % of the time; four
-// wavefronts per SIMD instead of three, 15 registers spilled: no faster).  Per
-// launch, exact, first order: tri 768^2 1,142 -> 1,035 us, tets 40^3 (a blast,
-// mostly at rest) 230 -> 150 us, quad 128^2 34.6 -> 29.2 us; VALU instructions
-// per wavefront 1,547 -> 1,264.
+// that share a divisor share its reciprocal (quot).  The velocities wait in LDS
+// during the iterations, so that four wavefronts per SIMD fit (5 registers
+// spilled) instead of three.  What bounds the sweep is latency between the
+// barriers and instruction issue (VALU about half of the time).  Per launch,
+// exact, first order: tri 768^2 1,142 -> 915 us, tets 40^3 (a blast, mostly at
+// rest) 230 -> 142 us, quad 128^2 34.6 -> 27.7 us; VALU instructions per
+// wavefront 1,547 -> about 1,260.  With three wavefronts and the velocities in
+// registers: 1,035, 150 and 29.2 us.
 //
 // Output: one row of six partial sums per node-sorted sub-element slot q
 // (vertex-major, so a group's rows are one contiguous run): P[6*q + k] = sum
@@ -65,17 +67,31 @@ SFV_DEV int xcd_block(int per_xcd) {
   return (b & 7) * per_xcd + (b >> 3);
 }
 
-// In-order sum row[b] + ... + row[e-1] starting from 0.0; loads are issued
-// eight at a time, the additions stay sequential (adding the +0.0 padding
-// leaves every partial sum unchanged).
+// In-order sum row[b] + ... + row[e-1] starting from 0.0: the loads of eight, four
+// and at most three entries are issued together, the additions stay sequential
+// (adding the +0.0 padding leaves every partial sum unchanged).
+template <int N>
+SFV_DEV double seg_add(double acc, const double *row) {
+  double t[N];
+#pragma unroll
+  for (int q = 0; q < N; q++) t[q] = row[q];
+#pragma unroll
+  for (int q = 0; q < N; q++) acc = acc + t[q];
+  return acc;
+}
 SFV_DEV double seg_sum(const double *row, int b, int e) {
   double acc = 0.0;
-  for (int j0 = b; j0 < e; j0 += 8) {
-    double t[8];
+  for (; b + 8 <= e; b += 8) acc = seg_add<8>(acc, row + b);
+  if (b + 4 <= e) {
+    acc = seg_add<4>(acc, row + b);
+    b += 4;
+  }
+  if (b < e) {
+    double t[3];
 #pragma unroll
-    for (int q = 0; q < 8; q++) t[q] = (j0 + q < e) ? row[j0 + q] : 0.0;
+    for (int q = 0; q < 3; q++) t[q] = (b + q < e) ? row[b + q] : 0.0;
 #pragma unroll
-    for (int q = 0; q < 8; q++) acc = acc + t[q];
+    for (int q = 0; q < 3; q++) acc = acc + t[q];
   }
   return acc;
 }
@@ -120,8 +136,12 @@ static __global__ __launch_bounds__(kGrpThreads) void k_sweep_order(DevMesh m) {
   m.ws_id[w] = (uint16_t)(tid | seg_of(vtab, nv, tid) << 8);
 }
 
+// nine rows of nodal terms and six of velocities put by during the iterations,
+// then twelve of fluxes; 15 rows leave room for four workgroups per CU
+constexpr int kFluxRows = 15;
+
 struct FluxLds {
-  double red[12][kRedStride];
+  double red[kFluxRows][kRedStride];
   double sum[kGrpVert][9];
   double vn[kGrpVert][3];
   double bp[kGrpVert][3];
@@ -274,6 +294,12 @@ SFV_DEV void node_flux_group(const FluxArgs &a, const double *__restrict__ U, in
     const double vn_l = wl[1] * n[0] + wl[2] * n[1] + wl[3] * n[2];
     const double vn_r = wr[1] * n[0] + wr[2] * n[1] + wr[3] * n[2];
     const double yal = recip_of(al), yar = recip_of(ar);
+    // the velocities are needed again for the flux only: kept in the thread's
+    // column of the free rows, 12 registers less in the iterations
+    for (int d = 0; d < 3; d++) {
+      L.red[9 + d][lid] = wl[1 + d];
+      L.red[12 + d][lid] = wr[1 + d];
+    }
     for (int iter = 1; iter <= 4; iter++) {
       const double l0 = lam_l, r0 = lam_r;
       double vs = vbar;
@@ -335,6 +361,10 @@ SFV_DEV void node_flux_group(const FluxArgs &a, const double *__restrict__ U, in
       }
       __syncthreads();
       for (int d = 0; d < 3; d++) v_node[d] = L.vn[vl][d];
+    }
+    for (int d = 0; d < 3; d++) {
+      wl[1 + d] = L.red[9 + d][lid];
+      wr[1 + d] = L.red[12 + d][lid];
     }
     if (a.vp && tid < nv)
       for (int d = 0; d < 3; d++) a.vp[d * m.V + vb + tid] = L.vn[tid][d];
@@ -482,7 +512,7 @@ static __global__ __launch_bounds__(256) void k_prim(long C, const double *__res
 }
 
 template <int SCHEME>
-__global__ __launch_bounds__(kGrpThreads, 3) void k_node_flux(FluxArgs a) {
+__global__ __launch_bounds__(kGrpThreads, 4) void k_node_flux(FluxArgs a) {
   __shared__ FluxLds L;
   const int lb = xcd_block(a.per_xcd);
   if (lb >= a.nblocks) return;  // uniform over the workgroup
