@@ -2756,20 +2756,20 @@ void launch_phase(subfv_batch *b, int n, int phase) {
   const int per_xcd = (b->total_g + 7) / 8;
   hipLaunchKernelGGL(k_node_flux_multi<S>, dim3(8 * per_xcd), dim3(kGrpThreads), 0, b->stream,
                      (const InstDesc *)b->d_desc, (const int *)b->d_gtab, b->total_g, per_xcd, phase);
-  hipLaunchKernelGGL(k_gather_multi, dim3(b->total_c), dim3(kCellThreads), 0, b->stream, (const InstDesc *)b->d_desc,
+  hipLaunchKernelGGL(k_gather_multi, dim3(8 * ((b->total_c + 7) / 8)), dim3(kCellThreads), 0, b->stream, (const InstDesc *)b->d_desc,
                      (const int *)b->d_ctab, b->total_c);
   if (b->fold) {
-    hipLaunchKernelGGL(k_update_multi<true>, dim3(b->total_c), dim3(kCellThreads), 0, b->stream,
+    hipLaunchKernelGGL(k_update_multi<true>, dim3(8 * ((b->total_c + 7) / 8)), dim3(kCellThreads), 0, b->stream,
                        (const InstDesc *)b->d_desc, (const int *)b->d_ctab, b->total_c, phase);
-    hipLaunchKernelGGL(k_finish_multi, dim3(b->total_c), dim3(kCellThreads), 0, b->stream,
+    hipLaunchKernelGGL(k_finish_multi, dim3(8 * ((b->total_c + 7) / 8)), dim3(kCellThreads), 0, b->stream,
                        (const InstDesc *)b->d_desc, (const int *)b->d_ctab, b->total_c, phase);
     return;
   }
   hipLaunchKernelGGL(k_finalize_dt_multi, dim3(n), dim3(kCellThreads), 0, b->stream, (const InstDesc *)b->d_desc);
-  hipLaunchKernelGGL(k_update_multi<false>, dim3(b->total_c), dim3(kCellThreads), 0, b->stream,
+  hipLaunchKernelGGL(k_update_multi<false>, dim3(8 * ((b->total_c + 7) / 8)), dim3(kCellThreads), 0, b->stream,
                      (const InstDesc *)b->d_desc, (const int *)b->d_ctab, b->total_c, phase);
   hipLaunchKernelGGL(k_finalize_omega_multi, dim3(n), dim3(kCellThreads), 0, b->stream, (const InstDesc *)b->d_desc);
-  hipLaunchKernelGGL(k_update_fixup_multi, dim3(b->total_c), dim3(kCellThreads), 0, b->stream,
+  hipLaunchKernelGGL(k_update_fixup_multi, dim3(8 * ((b->total_c + 7) / 8)), dim3(kCellThreads), 0, b->stream,
                      (const InstDesc *)b->d_desc, (const int *)b->d_ctab, b->total_c, phase);
 }
 
@@ -2928,7 +2928,7 @@ int subfv_batch_run(subfv_batch *b, subfv_ctx **ctxs, int32_t n, int32_t n_steps
   for (int i = 0; i < n; i++) fill_desc(ctxs[i], hd[i]);
   BHIP(b, hipMemcpyAsync(b->d_desc, hd.data(), n * sizeof(InstDesc), hipMemcpyHostToDevice, b->stream));
   if (n_steps > 0)
-    hipLaunchKernelGGL(k_prim_multi, dim3(b->total_c), dim3(kCellThreads), 0, b->stream, (const InstDesc *)b->d_desc,
+    hipLaunchKernelGGL(k_prim_multi, dim3(8 * ((b->total_c + 7) / 8)), dim3(kCellThreads), 0, b->stream, (const InstDesc *)b->d_desc,
                        (const int *)b->d_ctab, b->total_c);
   int s = 0;
   if (use_graph == 2 && n_steps > 0) {

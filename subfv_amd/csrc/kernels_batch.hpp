@@ -50,8 +50,9 @@ __global__ __launch_bounds__(kGrpThreads, 4) void k_node_flux_multi(const InstDe
 }
 
 __global__ __launch_bounds__(kCellThreads) void k_gather_multi(const InstDesc *d, const int *ctab, int total) {
-  if ((int)blockIdx.x >= total) return;
-  const int e = ctab[blockIdx.x];
+  const int lb = xcd_block((total + 7) / 8);  // neighbouring cells share their slots' lines
+  if (lb >= total) return;
+  const int e = ctab[lb];
   const InstDesc &D = *(const InstDesc *)((const CInstDesc *)d + (e >> kTabShift));
   if ((e & kTabMask) >= D.ncblk) return;
   gather_block(D.ga, e & kTabMask);
@@ -65,8 +66,9 @@ __global__ __launch_bounds__(kCellThreads) void k_finalize_dt_multi(const InstDe
 template <bool FOLD>
 __global__ __launch_bounds__(kCellThreads) void k_update_multi(const InstDesc *d, const int *ctab, int total,
                                                                int phase) {
-  if ((int)blockIdx.x >= total) return;
-  const int e = ctab[blockIdx.x];
+  const int lb = xcd_block((total + 7) / 8);  // neighbouring cells share their slots' lines
+  if (lb >= total) return;
+  const int e = ctab[lb];
   const InstDesc &D = *(const InstDesc *)((const CInstDesc *)d + (e >> kTabShift));
   if ((e & kTabMask) >= D.ncblk) return;
   update_block<kDiagNone, FOLD>(D.ua, D.U[(D.cur0 + phase) % 3], D.U[(D.cur0 + phase + 1) % 3], e & kTabMask);
@@ -74,8 +76,9 @@ __global__ __launch_bounds__(kCellThreads) void k_update_multi(const InstDesc *d
 
 // the primitives of every instance's current state
 __global__ __launch_bounds__(kCellThreads) void k_prim_multi(const InstDesc *d, const int *ctab, int total) {
-  if ((int)blockIdx.x >= total) return;
-  const int e = ctab[blockIdx.x];
+  const int lb = xcd_block((total + 7) / 8);  // neighbouring cells share their slots' lines
+  if (lb >= total) return;
+  const int e = ctab[lb];
   const InstDesc &D = *(const InstDesc *)((const CInstDesc *)d + (e >> kTabShift));
   if ((e & kTabMask) >= D.ncblk) return;
   prim_block(D.ua.m.C, D.U[D.cur0 % 3], D.ua.W, e & kTabMask);
@@ -84,8 +87,9 @@ __global__ __launch_bounds__(kCellThreads) void k_prim_multi(const InstDesc *d, 
 // k_finalize_omega_multi and k_update_fixup_multi in one (finish_block)
 __global__ __launch_bounds__(kCellThreads) void k_finish_multi(const InstDesc *d, const int *ctab, int total,
                                                                int phase) {
-  if ((int)blockIdx.x >= total) return;
-  const int e = ctab[blockIdx.x];
+  const int lb = xcd_block((total + 7) / 8);  // neighbouring cells share their slots' lines
+  if (lb >= total) return;
+  const int e = ctab[lb];
   const InstDesc &D = *(const InstDesc *)((const CInstDesc *)d + (e >> kTabShift));
   if ((e & kTabMask) >= D.ncblk) return;
   finish_block<kDiagNone>(D.ua, D.U[(D.cur0 + phase) % 3], D.U[(D.cur0 + phase + 1) % 3], e & kTabMask);
@@ -98,8 +102,9 @@ __global__ __launch_bounds__(kCellThreads) void k_finalize_omega_multi(const Ins
 
 __global__ __launch_bounds__(kCellThreads) void k_update_fixup_multi(const InstDesc *d, const int *ctab, int total,
                                                                      int phase) {
-  if ((int)blockIdx.x >= total) return;
-  const int e = ctab[blockIdx.x];
+  const int lb = xcd_block((total + 7) / 8);  // neighbouring cells share their slots' lines
+  if (lb >= total) return;
+  const int e = ctab[lb];
   const InstDesc &D = *(const InstDesc *)((const CInstDesc *)d + (e >> kTabShift));
   if ((e & kTabMask) >= D.ncblk) return;
   update_fixup_block<kDiagNone>(D.ua, D.U[(D.cur0 + phase) % 3], D.U[(D.cur0 + phase + 1) % 3], e & kTabMask);
