@@ -202,9 +202,9 @@ int subfv_compute_rhs_ns(subfv_ctx *ctx);
  * i = 1..n_bc (arrays 0-based): bc_v_id / bc_t_id 1 = neumann, 2 = dirichlet
  * (bc_type_V / bc_type_T), bc_val_v(3, n_bc), bc_val_t(n_bc).  Applies to
  * subfv_compute_rhs_ns (rhs and "diag") and to the stages of subfv_run.
- * Vertices may have at most 64 sub-faces and 64 sub-elements (a mesh whose
- * vertices all have at most 16 takes kernels with the setup's matrices in LDS;
- * others, e.g. tetrahedral meshes, keep them in a global workspace). */
+ * Vertices may have at most 64 sub-faces and 64 sub-elements; the sizes of the
+ * mesh's largest vertex choose the kernels and how its nodal inverses are
+ * stored. */
 int subfv_set_diffusion(subfv_ctx *ctx, int32_t activate, double mu_p, double cv_p, double prandtl,
                         int32_t n_bc, const int32_t *bc_v_id, const double *bc_val_v, const int32_t *bc_t_id,
                         const double *bc_val_t);
@@ -337,7 +337,8 @@ int subfv_bcsr_add_block(subfv_bcsr *A, int32_t i, int32_t j, const double *M);
  * subfv_run(ctx, n_steps, 0, ...) alone.  Members must share the device and
  * the scheme and run the first-order inviscid forward-Euler loop.
  * subfv_batch_run enqueues n_steps steps on the batch's stream and returns.
- * use_graph 0: six multi-instance launches per step; 1: whole 3-step cycles
+ * use_graph 0: four multi-instance launches per step (six where a member has
+ * more than 262,144 cells); 1: whole 3-step cycles
  * replay one captured hipGraph (re-captured when the membership changes);
  * 2: one persistent cooperative launch for all n_steps (a resident grid
  * with device-side work queues and grid barriers between the phases).

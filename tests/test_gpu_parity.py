@@ -241,3 +241,36 @@ def test_local_time_step_loop_bit_exact(solver, case):
     assert st == 0
     assert np.array_equal(got, ref), np.abs(got - ref).max()
     assert t == info["t"] and dt == info["dt"]
+
+
+@pytest.mark.parametrize("n", [512, 513])
+@pytest.mark.parametrize("ts,second_order", [(0, False), (1, True)])
+def test_stage_reductions_at_the_size_limit_bit_exact(solver, n, ts, second_order):
+    """512^2 cells are the most (1,024 blocks of 256) whose dt and omega
+    minima the update and its correction form themselves; 513^2 take the
+    kernels of their own.  Both give the oracle's bits, dt and time."""
+    print(f"[gpu] stage reductions {n} {ts}", flush=True)
+    mesh = mg.quad_mesh(n)
+    solver.build_mesh(mesh)
+    om = O.OracleMesh(mesh)
+    solver.set_config(make_config("two_wave", second_order=second_order, cfl=0.4))
+    solver.set_time(0.0)
+    cfg = O.make_config("two_wave", second_order=second_order, cfl=0.4)
+    sol = mg.init_1drp(om.elem_coord, 0.5, [1, 0.1, 0, 0, 1], [0.125, 0, 0, 0, 0.1])
+    solver.put_sol(sol)
+    t, _ = solver.run(2, ts)
+    st, ref, info = om.run(cfg, sol, 2, ts)
+    assert st == 0
+    assert np.array_equal(solver.get_sol(), ref)
+    assert t == info["t"]
+
+
+def test_geometry_of_one_cell_bit_exact(solver):
+    """One hexahedron: its arrays are larger than the partials that larger
+    meshes' outputs are rearranged in."""
+    print("[gpu] one cell", flush=True)
+    mesh = mg.hex_mesh(1)
+    solver.build_mesh(mesh)
+    om = O.OracleMesh(mesh)
+    for g in GEOM:
+        assert np.array_equal(solver.mesh_d(g), om.getd(g)), g

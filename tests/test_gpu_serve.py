@@ -133,3 +133,20 @@ def test_pooled_context_reused_for_a_different_mesh(requests, mode):
     for rid in a:
         assert np.array_equal(a[rid], m[rid]), rid
 
+
+@pytest.mark.parametrize("use_graph", [False, True])
+@pytest.mark.parametrize("side", [512, 513])
+def test_batch_with_a_large_member_equals_solves_alone(side, use_graph):
+    """A member above 1,024 blocks of cells takes the whole batch, small
+    members included, to the reductions' own kernels."""
+    print(f"[gpu] batch with {side}^2 cells graph={use_graph}", flush=True)
+    reqs = S.make_requests(n_req=4, rate=1e6, steps=7, cmin=8 ** 2, cmax=20 ** 2)
+    reqs[1].kind, reqs[1].n = "quad", side
+    reqs = S.prepare(reqs, workers=4)
+    alone, _ = S.serve_plain(reqs, keep=True, realtime=False)
+    mixed, _ = S.serve(reqs, S.Params(chunk=7, max_batch=4, use_graph=use_graph), keep=True, realtime=False)
+    a = {r.rid: r.sol for r in alone}
+    m = {r.rid: r.sol for r in mixed}
+    assert set(a) == set(m) == {r.rid for r in reqs}
+    for rid in a:
+        assert np.array_equal(a[rid], m[rid]), rid
