@@ -783,19 +783,9 @@ int ensure_diffusion(subfv_ctx *c) {
       off[v] = at | ni << 48 | tag << 56;
       at += 10 * nb;
     }
-    c->diff_lds = 0;
-    if (c->diff_cls != kDiffLarge) {
-      const int per = kDiffApplyVerts[c->diff_cls];
-      for (int v0 = 0; v0 < h.nv; v0 += per) {
-        int sum = 0;
-        // past the last vertex the lanes mirror it
-        for (int k = 0; k < per; k++) {
-          const int v = std::min(v0 + k, h.nv - 1);
-          sum += diff_apply_lds(st[v] & 0xFF, h.sf_off[v + 1] - h.sf_off[v]);
-        }
-        c->diff_lds = std::max(c->diff_lds, sum);
-      }
-    }
+    c->diff_lds = c->diff_cls == kDiffLarge ? 0 : apply_lds_wave(h.nv, kDiffApplyVerts[c->diff_cls], [&](long v) {
+      return apply_lds<false>(st[v] & 0xFF, h.sf_off[v + 1] - h.sf_off[v]);
+    });
     if ((r = room(fixed + sizeof(double) * at))) return r;
     if ((r = upload(c, &c->doff, off))) return r;
     if ((r = dalloc(c, &c->pre, (size_t)at))) return r;

@@ -747,11 +747,6 @@ __global__ __launch_bounds__(64) void k_visc(DiffArgs a) {
 // matrices took 4.88 ms per residual (19 GB, 4.6 TB/s); the inverses (4 GB)
 // staged in LDS, 9 wavefronts per CU, 2.66 ms; like this 1.46 ms, bound by
 // instruction issue (0.8 ms of it) and latency, 3.4 TB/s.
-template <bool GLOBAL>
-SFV_DEV __host__ int apply_lds(int ni, int nf) {
-  const int part = GLOBAL ? 8 * ni : (ni > 2 ? 4 * ni * ni : 8 * ni);
-  return (part + 4 * ni + 3 * nf + (ni + 1) / 2 + 1) & ~1;  // even: rows of four are read and written in pairs
-}
 SFV_DEV void put4(double *p, double a, double b, double c, double d) {
   ((double2 *)p)[0] = make_double2(a, b);
   ((double2 *)p)[1] = make_double2(c, d);
@@ -771,10 +766,12 @@ __global__ __launch_bounds__(256, 3) void k_visc_apply(DiffArgs a) {
   const DevMesh &m = a.m;
   const int lb = xcd_block(a.vper_xcd);  // neighbouring vertices share cells
   if (lb >= a.vblocks) return;
-  const int grp = threadIdx.x / LPV, lane = threadIdx.x % LPV;
-  const long v_ = (long)lb * (blockDim.x / LPV) + grp;
-  const bool live = v_ < m.V;
-  const long v = live ? v_ : m.V - 1;  // spare lanes mirror the last vertex and store nothing
+  constexpr int per = 64 / LPV;
+  const int lane = threadIdx.x % LPV, wave = threadIdx.x >> 6, grp = (threadIdx.x & 63) / LPV;
+  const long w = (long)lb * (blockDim.x >> 6) + wave;
+  const long v = apply_vertex(w, per, grp, m.V);
+  if (v < 0) return;  // uniform over the wavefront, which shares no barrier with the others
+  const bool live = w * per + grp < m.V;  // spare lanes mirror the last vertex and store nothing
   const int sf0 = m.sf_off[v], nf = m.sf_off[v + 1] - sf0;
   const int se0 = m.se_off[v], ns = m.se_off[v + 1] - se0;
   const uint64_t dd = a.doff[v];
@@ -792,13 +789,12 @@ __global__ __launch_bounds__(256, 3) void k_visc_apply(DiffArgs a) {
   SlotReg r;
   if (lane < ns) slot_load<false>(a, se0 + lane, r, mu0);
   // this vertex's LDS, behind those of the wavefront's earlier vertices
-  double *L = lds_all + (long)(threadIdx.x >> 6) * a.lds_stride;
+  double *L = lds_all + (long)wave * a.lds_stride;
   {
     const int size = apply_lds<GLOBAL>(ni, nf);
-    const int mine = (threadIdx.x & 63) / LPV;
-    for (int q = 0; q < 64 / LPV - 1; q++) {
+    for (int q = 0; q < per - 1; q++) {
       const int sq = __shfl(size, q * LPV);
-      if (q < mine) L += sq;
+      if (q < grp) L += sq;
     }
   }
   double *const fL = L;  // [ni][2][4] one-sided fluxes, then the block products [ni][ni][4]
@@ -1297,8 +1293,6 @@ hipError_t launch_diff_terms(int cls, DiffArgs a, hipStream_t s) {
 hipError_t launch_diff_gather(DiffArgs a, hipStream_t s) {
   return a.mu_cell ? launch_gather<kDiffSlot>(a, 1, 1, s) : launch_gather<kDiffRow>(a, 1, 0, s);
 }
-
-int diff_apply_lds(int ni, int nf) { return apply_lds<false>(ni, nf); }
 
 hipError_t launch_diff_expand(long C, const double *U, const double *dblk, double cv, double *diag, hipStream_t s) {
   hipLaunchKernelGGL(k_diff_expand, dim3((unsigned)((C + 255) / 256)), dim3(256), 0, s, C, U, dblk, cv, diag);

@@ -5,6 +5,7 @@
 // Parameters, arguments and launchers; the kernels are in diffusion.hip.
 #pragma once
 #include "device_mesh.hpp"
+#include "diff_plan.hpp"
 #include "kernels_flux.hpp"
 #include "physics.hpp"
 
@@ -47,18 +48,13 @@ struct DiffArgs {
   const uint8_t *fpos;     // [SF] a sub-face's place among its vertex's faces, with boundary flags
   int nim, nfm, nsm;       // largest stored faces, sub-faces and sub-elements of a vertex
   int lmat;                // doubles of LDS for the matrices a vertex forms (set by the launchers)
-  int lds_wave;            // doubles of LDS of the apply's fullest wavefront (diff_apply_lds of its vertices)
+  int lds_wave;            // doubles of LDS of the apply's fullest wavefront (apply_lds_wave)
   int vper_xcd, vblocks;   // XCD slices of the vertex blocks (apply)
   int cper_xcd, cblocks;   // and of the cell blocks (gather)
   int parts;               // apply: 1 momentum system, 2 heat system, 3 both
   int pivot;               // form the inverses with partial pivoting throughout
   int lds_stride;          // doubles of LDS per vertex, per wavefront in the apply (set by the launchers)
 };
-
-// doubles of LDS the constant-viscosity apply holds for a vertex of ni stored faces
-// and nf faces, and how many consecutive vertices share a wavefront
-int diff_apply_lds(int ni, int nf);
-constexpr int kDiffApplyVerts[2] = {4, 2};  // kDiffHalf, kDiffWave
 
 // stored faces and tags of every vertex, the faces' places and the slots' codes
 void launch_diff_tables(const DevMesh &m, int *vstat, uint8_t *fpos, uint32_t *scode, double *sivol, hipStream_t s);

@@ -160,17 +160,75 @@ def test_viscous_100_steps_within_1e12(solver, name, ts):
 @pytest.mark.parametrize("law", ["constant", "sutherland"])
 @pytest.mark.parametrize("k,layers", [(3, 1), (10, 1), (11, 1), (7, 2), (22, 1), (8, 2), (13, 2), (21, 2)])
 def test_vertex_size_classes_match_oracle(solver, k, layers, law):
-    """rhs and diag of one residual within 1e-12 of the viscous terms' scale,
-    as for the meshes above."""
     print(f"[gpu] viscous class fan k={k} layers={layers} {law}", flush=True)
-    mesh = fan_prism_mesh(k, layers)
+    viscous_matches_oracle(solver, fan_prism_mesh(k, layers), law, dict(boundary_2d=False), {})
+
+
+_FACES = {4: ([0, 1, 2], [0, 1, 3], [1, 2, 3], [0, 2, 3]),
+          5: ([0, 1, 2, 3], [4, 5, 6, 7], [0, 1, 5, 4], [1, 2, 6, 5], [2, 3, 7, 6], [3, 0, 4, 7]),
+          6: ([0, 1, 2], [3, 4, 5], [0, 1, 4, 3], [1, 2, 5, 4], [2, 0, 3, 5])}
+
+
+def tag_boundary(mesh, tag):
+    """The mesh with its boundary faces tagged: tag(centre) is 0 (untagged, the
+    default wall) or a BC index."""
+    off = mg.elem_offsets(mesh.kind)
+    seen = {}
+    for e, kind in enumerate(mesh.kind):
+        v = mesh.elem_vert[off[e]:off[e + 1]]
+        for f in _FACES[int(kind)]:
+            seen.setdefault(frozenset(v[f].tolist()), []).append(v[f])
+    nv, verts, tags = [], [], []
+    for f in seen.values():
+        t = tag(mesh.coord[f[0] - 1].mean(axis=0)) if len(f) == 1 else 0
+        if t:
+            nv.append(len(f[0]))
+            verts.append(f[0])
+            tags.append(t)
+    mesh.bf_nvert, mesh.bf_tag = np.array(nv, np.int32), np.array(tags, np.int32)
+    mesh.bf_vert = np.concatenate(verts).astype(np.int32)
+    return mesh
+
+
+def shell_mesh(k, rings):
+    """One layer of a spherical shell: k prisms around each pole, k hexahedra
+    in each of the rings - 1 belts between.  The numbering starts at one pole,
+    so the other, with its k sub-elements, is the last vertex."""
+    th = np.pi * (1 + np.arange(rings)) / (rings + 1)
+    ph = 2 * np.pi * np.arange(k) / k
+    ring = np.stack([np.outer(np.sin(th), np.cos(ph)), np.outer(np.sin(th), np.sin(ph)),
+                     np.outer(np.cos(th), np.ones(k))], -1).reshape(-1, 3)
+    pts = np.concatenate([[[0, 0, 1.0]], ring, [[0, 0, -1.0]]])
+    n, south = len(pts), len(pts) - 1
+    at = lambda r, q: 1 + r * k + q % k
+    ev, kind = [], []
+    for q in range(k):
+        for low in ([0, at(0, q), at(0, q + 1)], [south, at(rings - 1, q + 1), at(rings - 1, q)]):
+            ev.append(low + [v + n for v in low])
+            kind.append(6)
+        for r in range(rings - 1):
+            low = [at(r, q), at(r + 1, q), at(r + 1, q + 1), at(r, q + 1)]
+            ev.append(low + [v + n for v in low])
+            kind.append(5)
+    flat = np.concatenate([np.array(e) for e in ev]) + 1
+    return mg.Mesh(np.concatenate([pts, 1.3 * pts]), np.array(kind, np.int32), flat.astype(np.int32),
+                   boundary_2d=False, name="shell")
+
+
+TAGGED = (dict(boundary_2d=False, bcs=[("freestream", (1.0, 0.2, 0.0, 0.0, 1.0)), ("outflowsupersonic", (0,) * 5)]),
+          dict(bcs_v=[("dirichlet", (0.1, -0.05, 0.02)), ("neumann", (0, 0, 0))],
+               bcs_t=[("dirichlet", 1.5e-3), ("dirichlet", 1.2e-3)]))
+
+
+def viscous_matches_oracle(solver, mesh, law, cfgkw, dkw):
+    """rhs and diag of one first-order residual within 1e-12 of the viscous
+    terms' scale, as for the meshes above."""
     solver.build_mesh(mesh)
     om = O.OracleMesh(mesh)
     suth = law == "sutherland"
     sol = warm_state(om.elem_coord) if suth else smooth_state(om.elem_coord)
-    kw = dict(boundary_2d=False, second_order=False)
-    solver.set_config(make_config("multi_point", **kw))
-    solver.set_diffusion(True, mu=2e-3)
+    solver.set_config(make_config("multi_point", second_order=False, **cfgkw))
+    solver.set_diffusion(True, mu=2e-3, **dkw)
     solver.set_sutherland(suth)
     try:
         solver.put_sol(sol)
@@ -179,13 +237,25 @@ def test_vertex_size_classes_match_oracle(solver, k, layers, law):
     finally:
         solver.set_sutherland(False)
         solver.set_diffusion(False)
-    ocfg = O.make_config("multi_point", diffusion=True, mu=2e-3, sutherland=suth, **kw)
+    ocfg = O.make_config("multi_point", second_order=False, diffusion=True, mu=2e-3, sutherland=suth, **cfgkw, **dkw)
     r0, _ = om.compute_euler_flux(ocfg, sol)
     rd, dd = om.add_diffusion(ocfg, sol)
     scale = np.abs(rd).max(axis=0) + 1e-300
     assert np.all(np.abs(rhs - (r0 + rd)) <= 1e-12 * scale[None, :] + 1e-14 * np.abs(r0 + rd)), \
         np.abs(rhs - r0 - rd).max(axis=0) / scale
     assert np.abs(diag - dd).max() <= 1e-12 * np.abs(dd).max()
+
+
+@pytest.mark.parametrize("law", ["constant", "sutherland"])
+@pytest.mark.parametrize("k,rings", [(8, 2), (10, 4), (13, 3)])
+def test_largest_vertex_last_matches_oracle(solver, k, rings, law):
+    """A tagged pole as the last vertex, larger than those before it: the
+    wavefronts that round the launch up to whole workgroups lie past it."""
+    print(f"[gpu] viscous shell k={k} rings={rings} {law}", flush=True)
+    mesh = tag_boundary(shell_mesh(k, rings), lambda x: 1 if x[2] < -0.8 and x[0] > 0.0 and abs(x[1]) < 0.3 else 0)
+    n_faces = O.OracleMesh(mesh).geti("vert_n_sub_faces")
+    assert n_faces[-1] == n_faces.max() and -(-n_faces.size // 16) * 4 > -(-n_faces.size // 4)
+    viscous_matches_oracle(solver, mesh, law, *TAGGED)
 
 
 def test_vertices_beyond_the_limit_are_rejected(solver):
