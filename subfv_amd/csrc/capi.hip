@@ -150,6 +150,11 @@ struct subfv_ctx {
   int diff_cls = 0;  // DiffClass of the mesh
   int diff_nim = 0, diff_nfm = 0, diff_nsm = 0, diff_lds = 0;  // a vertex's largest sizes (DiffArgs)
   long pre_n = 0;  // doubles in the packed inverses
+  // rearranges component arrays on their way to and from the host, a piece at a
+  // time: no other buffer is written, so a read disturbs no work in flight
+  std::mutex io_mu;
+  double *io = nullptr;
+  long io_n = 0;
   int *derr = nullptr;  // [2]: error bits of the path, failed check_mesh cells
   StepState *st = nullptr;
   double host_t = 0.0;
@@ -949,28 +954,50 @@ int mesh_i32(const subfv::HostMesh &h, const char *name, int32_t *out, int64_t c
   return (int64_t)v.size();
 }
 
-// [ncomp][n] on the device to the reference's [n][ncomp] and back; one lane per
-// interleaved value
-__global__ __launch_bounds__(256) void k_interleave(int ncomp, long n, const double *soa, double *aos) {
+// Elements i0 .. i0 + m of [ncomp][n] on the device to the reference's [n][ncomp]
+// and back; one lane per interleaved value
+__global__ __launch_bounds__(256) void k_interleave(int ncomp, long n, long i0, long m, const double *soa, double *aos) {
   const long q = (long)blockIdx.x * 256 + threadIdx.x;
-  if (q < ncomp * n) aos[q] = soa[(q % ncomp) * n + q / ncomp];
+  if (q < ncomp * m) aos[q] = soa[(q % ncomp) * n + i0 + q / ncomp];
 }
-__global__ __launch_bounds__(256) void k_deinterleave(int ncomp, long n, const double *aos, double *soa) {
+__global__ __launch_bounds__(256) void k_deinterleave(int ncomp, long n, long i0, long m, const double *aos,
+                                                      double *soa) {
   const long q = (long)blockIdx.x * 256 + threadIdx.x;
-  if (q < ncomp * n) soa[(q % ncomp) * n + q / ncomp] = aos[q];
+  if (q < ncomp * m) soa[(q % ncomp) * n + i0 + q / ncomp] = aos[q];
+}
+
+// Elements per piece through c->io, which grows to `need` doubles or to kIoDoubles
+// (8 MB); 0 where the device has no room for it.  The caller holds io_mu.
+constexpr long kIoDoubles = 1 << 20;
+long io_piece(subfv_ctx *c, int ncomp, long n) {
+  const long need = std::min(ncomp * n, kIoDoubles);
+  if (c->io_n < need) {
+    void *q = nullptr;
+    if (hipSetDevice(c->device) != hipSuccess || hipMalloc(&q, need * sizeof(double)) != hipSuccess) {
+      (void)hipGetLastError();
+    } else {
+      if (c->io) (void)hipFree(c->io);
+      c->io = (double *)q;
+      c->io_n = need;
+    }
+  }
+  return c->io_n / ncomp;
 }
 
 // Device arrays to and from host memory in the reference's layout: copied
 // straight between the device and the caller's array (a 2.1M-cell state: 8 ms
 // out into fresh pages and 3 ms in, where a vector in between and a host loop
-// took 55 ms), component arrays interleaved on the device first.  c->P, the node
-// sweep's partials, is free outside a residual and holds them where it is large
-// enough (8 values per sub-element: 5 per cell and 3 per vertex always fit, 3
-// per sub-face on all but meshes of a few cells).
-bool fits_partials(const subfv_ctx *c, int ncomp, long n) { return ncomp * n <= kSlotStride * c->dm.SE; }
-
+// took 55 ms), component arrays interleaved on the device first, or on the host
+// where the device has no room.
 int dev_to_host_soa(subfv_ctx *c, const double *d, int ncomp, long n, double *out) {
-  if (ncomp > 1 && !fits_partials(c, ncomp, n)) {
+  if (ncomp == 1) {
+    HIPCHK(c, hipMemcpyAsync(out, d, sizeof(double) * n, hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    return 0;
+  }
+  std::lock_guard<std::mutex> lk(c->io_mu);
+  const long piece = io_piece(c, ncomp, n);
+  if (!piece) {
     std::vector<double> tmp((size_t)ncomp * n);
     HIPCHK(c, hipMemcpyAsync(tmp.data(), d, tmp.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -978,23 +1005,37 @@ int dev_to_host_soa(subfv_ctx *c, const double *d, int ncomp, long n, double *ou
       for (int k = 0; k < ncomp; k++) out[(size_t)i * ncomp + k] = tmp[(size_t)k * n + i];
     return 0;
   }
-  if (ncomp > 1) {
-    hipLaunchKernelGGL(k_interleave, dim3(nblk(ncomp * n, 256)), dim3(256), 0, c->stream, ncomp, n, d, c->P);
+  for (long i0 = 0; i0 < n; i0 += piece) {
+    const long m = std::min(piece, n - i0);
+    hipLaunchKernelGGL(k_interleave, dim3(nblk(ncomp * m, 256)), dim3(256), 0, c->stream, ncomp, n, i0, m, d, c->io);
     HIPCHK(c, hipGetLastError());
-    d = c->P;
+    HIPCHK(c, hipMemcpyAsync(out + ncomp * i0, c->io, sizeof(double) * ncomp * m, hipMemcpyDeviceToHost, c->stream));
   }
-  HIPCHK(c, hipMemcpyAsync(out, d, sizeof(double) * ncomp * n, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   return 0;
 }
 
 int host_to_dev_soa(subfv_ctx *c, const double *in, int ncomp, long n, double *d) {
-  if (ncomp > 1 && !fits_partials(c, ncomp, n)) return fail(c, SUBFV_E_INVALID, "more values than the mesh holds");
-  double *to = ncomp > 1 ? c->P : d;
-  HIPCHK(c, hipMemcpyAsync(to, in, sizeof(double) * ncomp * n, hipMemcpyHostToDevice, c->stream));
-  if (ncomp > 1) {
-    hipLaunchKernelGGL(k_deinterleave, dim3(nblk(ncomp * n, 256)), dim3(256), 0, c->stream, ncomp, n,
-                       (const double *)to, d);
+  if (ncomp == 1) {
+    HIPCHK(c, hipMemcpyAsync(d, in, sizeof(double) * n, hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    return 0;
+  }
+  std::lock_guard<std::mutex> lk(c->io_mu);
+  const long piece = io_piece(c, ncomp, n);
+  if (!piece) {
+    std::vector<double> tmp((size_t)ncomp * n);
+    for (long i = 0; i < n; i++)
+      for (int k = 0; k < ncomp; k++) tmp[(size_t)k * n + i] = in[(size_t)i * ncomp + k];
+    HIPCHK(c, hipMemcpyAsync(d, tmp.data(), tmp.size() * sizeof(double), hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    return 0;
+  }
+  for (long i0 = 0; i0 < n; i0 += piece) {
+    const long m = std::min(piece, n - i0);
+    HIPCHK(c, hipMemcpyAsync(c->io, in + ncomp * i0, sizeof(double) * ncomp * m, hipMemcpyHostToDevice, c->stream));
+    hipLaunchKernelGGL(k_deinterleave, dim3(nblk(ncomp * m, 256)), dim3(256), 0, c->stream, ncomp, n, i0, m,
+                       (const double *)c->io, d);
     HIPCHK(c, hipGetLastError());
   }
   HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -1079,6 +1120,7 @@ void subfv_destroy(subfv_ctx *c) {
   c->chunks.clear();
   for (auto &ph : c->pins) (void)hipHostFree(ph.first);
   c->pins.clear();
+  if (c->io) (void)hipFree(c->io);
   if (c->derr) (void)hipFree(c->derr);
   if (c->st) (void)hipFree(c->st);
   if (c->ev) (void)hipEventDestroy(c->ev);

@@ -266,11 +266,29 @@ def test_stage_reductions_at_the_size_limit_bit_exact(solver, n, ts, second_orde
 
 
 def test_geometry_of_one_cell_bit_exact(solver):
-    """One hexahedron: its arrays are larger than the partials that larger
-    meshes' outputs are rearranged in."""
+    """One hexahedron: the smallest arrays."""
     print("[gpu] one cell", flush=True)
     mesh = mg.hex_mesh(1)
     solver.build_mesh(mesh)
     om = O.OracleMesh(mesh)
     for g in GEOM:
         assert np.array_equal(solver.mesh_d(g), om.getd(g)), g
+
+
+def test_arrays_longer_than_a_rearranged_piece_bit_exact(solver):
+    """Component arrays are rearranged 2^20 values at a time on their way to
+    and from the host: 460^2 cells' five residual components take two pieces,
+    their sub-face normals ten."""
+    print("[gpu] arrays in pieces", flush=True)
+    mesh = mg.quad_mesh(460)
+    solver.build_mesh(mesh)
+    om = O.OracleMesh(mesh)
+    solver.set_config(make_config("multi_point"))
+    sol = mg.vortex_state(om.elem_coord)
+    rhs, sl = solver.compute_euler_flux(sol)
+    r_rhs, r_sl = om.compute_euler_flux(O.make_config("multi_point"), sol)
+    assert np.array_equal(rhs, r_rhs)
+    assert np.array_equal(solver.mesh_d("sub_face_norm"), om.getd("sub_face_norm"))
+    other = rhs[::-1].copy()
+    solver.put("rhs", other)
+    assert np.array_equal(solver.get("rhs"), other)

@@ -150,3 +150,31 @@ def test_batch_with_a_large_member_equals_solves_alone(side, use_graph):
     assert set(a) == set(m) == {r.rid for r in reqs}
     for rid in a:
         assert np.array_equal(a[rid], m[rid]), rid
+
+
+def test_reading_a_member_leaves_a_running_batch_alone():
+    """Mesh arrays of a member read while its batch runs: the values of an idle
+    context, and the batch's states as without the reads."""
+    print("[gpu] batch with reads", flush=True)
+    reqs = S.prepare(S.make_requests(n_req=4, rate=1e6, steps=90, cmin=100 ** 2, cmax=160 ** 2), workers=4)
+    solvers = [S.Solver(0) for _ in reqs]
+    batch = S.Batch(0)
+    states, norms = [], []
+    try:
+        for reads in (0, 3):
+            for s, r in zip(solvers, reqs):
+                S.admit(s, r)
+            idle = [s.mesh_d("sub_face_norm") for s in solvers]
+            batch.run(solvers, 90, 0)
+            for _ in range(reads):
+                norms.append([s.mesh_d("sub_face_norm") for s in solvers])
+            batch.wait()
+            states.append([s.get_sol() for s in solvers])
+        for a, b in zip(*states):
+            assert np.array_equal(a, b)
+        for got in norms:
+            assert all(np.array_equal(a, b) for a, b in zip(got, idle))
+    finally:
+        batch.close()
+        for s in solvers:
+            s.close()
