@@ -124,9 +124,23 @@ def admit(s: Solver, r: Request, connectivity: str = "device"):
     s.set_time(0.0)
 
 
+# HBM per element by gmsh kind (hexahedron, prism, tetrahedron, pyramid) of an
+# instance's mesh, partials, states, primitives and work arrays.  Hexahedra and
+# prisms as in one-layer meshes, the larger per element: 4,234 and 3,197 bytes of
+# arrays, and up to a fifth more for the unused ends of the context's chunks
+# (measured: quads up to 5,029, triangles 3,931, tetrahedra 2,303, hexahedra of
+# 3-D meshes 3,840).
+BYTES_PER_ELEMENT = {5: 5100, 6: 3950, 4: 2400, 7: 3900}
+
+
 def device_bytes(r: Request) -> int:
-    """HBM an admitted instance holds (mesh, partials, states, work arrays)."""
-    return 3200 * r.cells + (4 << 20)
+    """HBM an admitted instance holds."""
+    if r.mesh is None:  # as the largest kind
+        per = BYTES_PER_ELEMENT[5] * r.cells
+    else:
+        n = np.bincount(r.mesh.kind, minlength=8)
+        per = sum(b * int(n[k]) for k, b in BYTES_PER_ELEMENT.items())
+    return per + (4 << 20)
 
 
 class Batch:

@@ -178,3 +178,24 @@ def test_reading_a_member_leaves_a_running_batch_alone():
         batch.close()
         for s in solvers:
             s.close()
+
+
+@pytest.mark.parametrize("mk", [lambda: mg.quad_mesh(20), lambda: mg.quad_mesh(128), lambda: mg.quad_mesh(420),
+                                lambda: mg.tri_mesh(128), lambda: mg.tri_mesh(300), lambda: mg.tet_mesh(24),
+                                lambda: mg.hex_mesh(40)],
+                         ids=["quad20", "quad128", "quad420", "tri128", "tri300", "tet24", "hex40"])
+def test_admission_estimate_covers_what_an_instance_holds(mk):
+    mesh = mk()
+    print(f"[gpu] admission estimate {mesh.name}", flush=True)
+    r = S.make_requests(n_req=1)[0]
+    r.mesh, r.cells, r.boundary_2d = mesh, mesh.n_elems, mesh.boundary_2d
+    s, batch = S.Solver(0), S.Batch(0)
+    try:
+        S.admit(s, r)
+        batch.run([s], 3, 0)
+        batch.wait()
+        held = s.count("device_bytes_used")
+    finally:
+        batch.close()
+        s.close()
+    assert held <= S.device_bytes(r) <= 1.4 * held + (4 << 20)
