@@ -207,6 +207,21 @@ int upload(subfv_ctx *c, T **p, const std::vector<T> &v) {
   return 0;
 }
 
+// Gives back what was taken from the chunks since, unless kept: a call that
+// fails half way leaves the context as it found it.
+struct ChunkMark {
+  subfv_ctx *c;
+  size_t i, off;
+  bool kept = false;
+  explicit ChunkMark(subfv_ctx *ctx) : c(ctx), i(ctx->chunk_i), off(ctx->chunk_off) {}
+  ~ChunkMark() {
+    if (kept) return;
+    (void)hipStreamSynchronize(c->stream);
+    c->chunk_i = i;
+    c->chunk_off = off;
+  }
+};
+
 // Host-to-device copy queued on the context's stream from its pinned
 // staging blocks (a plain memcpy into pinned memory, then an asynchronous
 // DMA copy); the blocks are reused from the start by the next upload, after
@@ -730,80 +745,106 @@ DiffArgs diff_args(subfv_ctx *c) {
 }
 
 // Once per mesh: the kernels' tables, each vertex's place in the packed
-// inverses, and the size class; once per mesh and parameter set with a
-// constant viscosity: the inverses of the nodal systems.
+// inverses, the size class and the buffers, whose sizes depend on the mesh only.
+// A failure takes nothing.
+int diffusion_buffers(subfv_ctx *c) {
+  const subfv::HostMesh &h = *c->hmp;
+  int r;
+  int mf = 1, me = 1;
+  for (int v = 0; v < h.nv; v++) {
+    const int nf = h.sf_off[v + 1] - h.sf_off[v], ns = h.v_seoff[v + 1] - h.v_seoff[v];
+    if (nf > kDiffMaxSub || ns > kDiffMaxSub)
+      return fail(c, SUBFV_E_INVALID, "viscous terms: vertex " + std::to_string(v + 1) + " has more than " +
+                                          std::to_string(kDiffMaxSub) + " sub-faces or sub-elements");
+    mf = std::max(mf, nf);
+    me = std::max(me, ns);
+  }
+  const size_t tables = 4ull * h.nv + h.nsf + 12ull * h.nse;
+  const size_t work = sizeof(double) * (h.nv + (size_t)kDiffSlot * h.nse + (29ull + kDiffBlk) * h.ne);
+  auto room = [&](size_t need) -> int {
+    size_t free_b = 0, total_b = 0;
+    HIPCHK(c, hipMemGetInfo(&free_b, &total_b));
+    if (need + ((size_t)1 << 30) > free_b)
+      return fail(c, SUBFV_E_DEVICE, "viscous terms: " + std::to_string(need >> 20) + " MiB needed, " +
+                                         std::to_string(free_b >> 20) + " MiB free");
+    return 0;
+  };
+  if ((r = room(tables + work))) return r;
+  ChunkMark mark(c);
+  int *vstat = nullptr;
+  uint8_t *fpos = nullptr;
+  uint32_t *scode = nullptr;
+  double *sivol = nullptr, *pre = nullptr, *PD = nullptr, *rdiff = nullptr, *dblk = nullptr, *diag = c->diag;
+  uint64_t *doff = nullptr;
+  if ((r = dalloc(c, &vstat, (size_t)h.nv))) return r;
+  if ((r = dalloc(c, &fpos, (size_t)h.nsf))) return r;
+  if ((r = dalloc(c, &scode, (size_t)h.nse))) return r;
+  if ((r = dalloc(c, &sivol, (size_t)h.nse))) return r;
+  launch_diff_tables(c->dm, vstat, fpos, scode, sivol, c->stream);
+  HIPCHK(c, hipGetLastError());
+  std::vector<int> st(h.nv);
+  HIPCHK(c, hipMemcpyAsync(st.data(), vstat, sizeof(int) * h.nv, hipMemcpyDeviceToHost, c->stream));
+  HIPCHK(c, hipStreamSynchronize(c->stream));
+  int nim = 1;
+  for (int v = 0; v < h.nv; v++) nim = std::max(nim, st[v] & 0xFF);
+  // 32 lanes per vertex hold a row of its inverse each (3 stored faces x 3
+  // <= 30 rows) while it is formed, 64 lanes up to 63 rows
+  c->diff_cls = nim <= 10 && me <= 16 ? kDiffHalf : (nim <= 21 ? kDiffWave : kDiffLarge);
+  c->diff_nim = nim;
+  c->diff_nfm = mf;
+  c->diff_nsm = me;
+  // doubles of each vertex's inverses: 3x3 blocks and heat entries on and
+  // below the diagonal, or all where the vertex is tagged; the large class
+  // reserves all (its inverses for cell viscosities are stored too)
+  std::vector<uint64_t> off(h.nv);
+  uint64_t at = 0;
+  for (int v = 0; v < h.nv; v++) {
+    const uint64_t ni = st[v] & 0xFF, tag = st[v] >> 8;
+    const uint64_t nb = tag || c->diff_cls == kDiffLarge ? ni * ni : ni * (ni + 1) / 2;
+    off[v] = at | ni << 48 | tag << 56;
+    at += 10 * nb;
+  }
+  c->diff_lds = c->diff_cls == kDiffLarge ? 0 : apply_lds_wave(h.nv, kDiffApplyVerts[c->diff_cls], [&](long v) {
+    return apply_lds<false>(st[v] & 0xFF, h.sf_off[v + 1] - h.sf_off[v]);
+  });
+  if ((r = room(work + sizeof(double) * at))) return r;
+  if ((r = upload(c, &doff, off))) return r;
+  if ((r = dalloc(c, &pre, (size_t)at))) return r;
+  if ((r = dalloc(c, &PD, (size_t)kDiffSlot * h.nse))) return r;
+  if ((r = dalloc(c, &rdiff, 4ull * h.ne))) return r;
+  if ((r = dalloc(c, &dblk, (size_t)kDiffBlk * h.ne))) return r;
+  if (!diag && (r = dalloc(c, &diag, 25ull * h.ne))) return r;
+  mark.kept = true;
+  c->pre_n = (long)at;
+  c->doff = doff;
+  c->pre = pre;
+  c->PD = PD;
+  c->rdiff = rdiff;
+  c->dblk = dblk;
+  c->diag = diag;
+  c->dfpos = fpos;
+  c->dscode = scode;
+  c->dsivol = sivol;
+  return 0;
+}
+
+// the cell viscosity buffers (and, past the blocks' minima, mu0corr), once per mesh
+int ensure_mu_buffers(subfv_ctx *c) {
+  int r;
+  if (!c->mu_cell && (r = dalloc(c, &c->mu_cell, (size_t)c->dm.C))) return r;
+  if (!c->mu_blk && (r = dalloc(c, &c->mu_blk, (size_t)nblk(c->dm.C, kCellThreads) + 1))) return r;
+  return 0;
+}
+
+// The buffers, once per mesh; once per mesh and parameter set with a constant
+// viscosity: the inverses of the nodal systems.
 int ensure_diffusion(subfv_ctx *c) {
   if (c->diff_ready) return 0;
   const subfv::HostMesh &h = *c->hmp;
   if (h.periodic) return fail(c, SUBFV_E_INVALID, "viscous terms are not available on periodic meshes");
   int r;
-  // the buffers' sizes depend on the mesh only: allocated once per mesh and
-  // kept when the viscous parameters change (a new mesh resets them)
-  if (!c->doff) {
-    int mf = 1, me = 1;
-    for (int v = 0; v < h.nv; v++) {
-      const int nf = h.sf_off[v + 1] - h.sf_off[v], ns = h.v_seoff[v + 1] - h.v_seoff[v];
-      if (nf > kDiffMaxSub || ns > kDiffMaxSub)
-        return fail(c, SUBFV_E_INVALID, "viscous terms: vertex " + std::to_string(v + 1) + " has more than " +
-                                            std::to_string(kDiffMaxSub) + " sub-faces or sub-elements");
-      mf = std::max(mf, nf);
-      me = std::max(me, ns);
-    }
-    const size_t fixed = sizeof(double) * ((size_t)(kDiffSlot + 2) * h.nse + (29ull + kDiffBlk) * h.ne + 2ull * h.nv) + h.nsf;
-    auto room = [&](size_t need) -> int {
-      size_t free_b = 0, total_b = 0;
-      HIPCHK(c, hipMemGetInfo(&free_b, &total_b));
-      if (need + ((size_t)1 << 30) > free_b)
-        return fail(c, SUBFV_E_DEVICE, "viscous terms: " + std::to_string(need >> 20) + " MiB needed, " +
-                                           std::to_string(free_b >> 20) + " MiB free");
-      return 0;
-    };
-    if ((r = room(fixed))) return r;
-    int *vstat = nullptr;
-    if ((r = dalloc(c, &vstat, (size_t)h.nv))) return r;
-    if ((r = dalloc(c, &c->dfpos, (size_t)h.nsf))) return r;
-    if ((r = dalloc(c, &c->dscode, (size_t)h.nse))) return r;
-    if ((r = dalloc(c, &c->dsivol, (size_t)h.nse))) return r;
-    launch_diff_tables(c->dm, vstat, c->dfpos, c->dscode, c->dsivol, c->stream);
-    HIPCHK(c, hipGetLastError());
-    std::vector<int> st(h.nv);
-    HIPCHK(c, hipMemcpyAsync(st.data(), vstat, sizeof(int) * h.nv, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    int nim = 1;
-    for (int v = 0; v < h.nv; v++) nim = std::max(nim, st[v] & 0xFF);
-    // 32 lanes per vertex hold a row of its inverse each (3 stored faces x 3
-    // <= 30 rows) while it is formed, 64 lanes up to 63 rows
-    c->diff_cls = nim <= 10 && me <= 16 ? kDiffHalf : (nim <= 21 ? kDiffWave : kDiffLarge);
-    c->diff_nim = nim;
-    c->diff_nfm = mf;
-    c->diff_nsm = me;
-    // doubles of each vertex's inverses: 3x3 blocks and heat entries on and
-    // below the diagonal, or all where the vertex is tagged; the large class
-    // reserves all (its inverses for cell viscosities are stored too)
-    std::vector<uint64_t> off(h.nv);
-    uint64_t at = 0;
-    for (int v = 0; v < h.nv; v++) {
-      const uint64_t ni = st[v] & 0xFF, tag = st[v] >> 8;
-      const uint64_t nb = tag || c->diff_cls == kDiffLarge ? ni * ni : ni * (ni + 1) / 2;
-      off[v] = at | ni << 48 | tag << 56;
-      at += 10 * nb;
-    }
-    c->diff_lds = c->diff_cls == kDiffLarge ? 0 : apply_lds_wave(h.nv, kDiffApplyVerts[c->diff_cls], [&](long v) {
-      return apply_lds<false>(st[v] & 0xFF, h.sf_off[v + 1] - h.sf_off[v]);
-    });
-    if ((r = room(fixed + sizeof(double) * at))) return r;
-    if ((r = upload(c, &c->doff, off))) return r;
-    if ((r = dalloc(c, &c->pre, (size_t)at))) return r;
-    c->pre_n = (long)at;
-    if ((r = dalloc(c, &c->PD, (size_t)kDiffSlot * h.nse))) return r;
-    if ((r = dalloc(c, &c->rdiff, 4ull * h.ne))) return r;
-    if ((r = dalloc(c, &c->dblk, (size_t)kDiffBlk * h.ne))) return r;
-  }
-  if (c->dparams.suth && !c->mu_cell) {
-    if ((r = dalloc(c, &c->mu_cell, (size_t)h.ne))) return r;
-    if ((r = dalloc(c, &c->mu_blk, (size_t)nblk(h.ne, kCellThreads) + 1))) return r;
-  }
-  if (!c->diag && (r = dalloc(c, &c->diag, 25ull * h.ne))) return r;
+  if (!c->doff && (r = diffusion_buffers(c))) return r;
+  if (c->dparams.suth && (r = ensure_mu_buffers(c))) return r;
   HIPCHK(c, hipMemsetAsync(c->diag, 0, sizeof(double) * 25 * h.ne, c->stream));
   HIPCHK(c, hipMemsetAsync(c->rdiff, 0, sizeof(double) * 4 * h.ne, c->stream));
   // with Sutherland's law the inverses depend on the state: formed per residual
@@ -1727,14 +1768,6 @@ int subfv_set_sutherland(subfv_ctx *c, int32_t activate, double mu0, double T0) 
     c->dparams = p;
     c->diff_ready = false;
   }
-  return 0;
-}
-
-// the cell viscosity buffers (and, past the blocks' minima, mu0corr), once per mesh
-int ensure_mu_buffers(subfv_ctx *c) {
-  int r;
-  if (!c->mu_cell && (r = dalloc(c, &c->mu_cell, (size_t)c->dm.C))) return r;
-  if (!c->mu_blk && (r = dalloc(c, &c->mu_blk, (size_t)nblk(c->dm.C, kCellThreads) + 1))) return r;
   return 0;
 }
 

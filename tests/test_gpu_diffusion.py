@@ -8,6 +8,10 @@ relative (measured: 1e-15 on tri, quad, 3-D hex and a 10-sub-element fan).
 Tetrahedral meshes (36 sub-faces and 24 sub-elements at an interior vertex)
 take the large-class kernels: inverses formed by a workgroup per vertex and
 read from HBM."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -483,3 +487,75 @@ def test_compute_mu_sutherland_matches_oracle(solver):
     rd, dd = om.add_diffusion(ocfg, sol)
     assert np.abs(r - rd).max() <= 1e-12 * np.abs(rd).max()
     assert np.abs(d - dd).max() <= 1e-12 * np.abs(dd).max()
+
+
+_MEMINFO = """
+#include <stddef.h>
+size_t free_now = 0;  /* 0: plenty */
+int hipMemGetInfo(size_t *f, size_t *t) {
+  *t = (size_t)1 << 38;
+  *f = free_now ? free_now : *t;
+  return 0;
+}
+"""
+
+_RETRY = """
+import ctypes, sys
+sys.path[:0] = {path!r}
+info = ctypes.CDLL({so!r}, mode=ctypes.RTLD_GLOBAL)  # before the library, whose calls it answers
+free_now = ctypes.c_size_t.in_dll(info, "free_now")
+import numpy as np
+from subfv_amd import meshgen as mg
+from subfv_amd.api import Solver, SubfvError, make_config
+from test_gpu_diffusion import smooth_state
+
+def rhs(s, sol):
+    s.put_sol(sol)
+    s.compute_rhs_ns()
+    return s.get("rhs")
+
+s = Solver(0)
+s.build_mesh(mg.tri_mesh(60))
+s.set_config(make_config("multi_point"))
+s.set_diffusion(True, mu=2e-3)
+sol = smooth_state(s.elem_coord)
+used = s.count("device_bytes_used")
+V, SF, SE, C = s.n_vert, s.n_sub_faces, s.n_sub_elems, s.n_elems
+# room for the tables and the work arrays, not for the inverses behind them
+free_now.value = (1 << 30) + 4 * V + SF + 12 * SE + 8 * (V + 16 * SE + 39 * C) + (1 << 20)
+for _ in range(3):
+    try:
+        rhs(s, sol)
+        raise AssertionError("accepted")
+    except SubfvError as e:
+        assert "MiB needed" in str(e), e
+    # (the work arrays of the inviscid residual before it aside)
+    held = s.count("device_bytes_used")
+    first = locals().get("first", held)
+    assert held == first, (held, first)
+free_now.value = 0
+got = rhs(s, sol)
+grown = s.count("device_bytes_used")
+t = Solver(0)
+t.build_mesh(mg.tri_mesh(60))
+t.set_config(make_config("multi_point"))
+t.set_diffusion(True, mu=2e-3)
+assert np.array_equal(rhs(t, sol), got)
+assert t.count("device_bytes_used") == grown, (t.count("device_bytes_used"), grown)
+print("RETRY_OK", used, first, grown)
+"""
+
+
+def test_failed_viscous_setup_takes_nothing(tmp_path):
+    """Viscous residuals refused for want of device memory, after the tables
+    were formed: each attempt gives back what it took, and with room again the
+    residual and the memory held are those of a context that never failed."""
+    print("[gpu] viscous setup without room", flush=True)
+    src, so = tmp_path / "meminfo.c", tmp_path / "libmeminfo.so"
+    src.write_text(_MEMINFO)
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(so), str(src)], check=True)
+    here = os.path.dirname(os.path.abspath(__file__))
+    path = [os.path.dirname(here), here, os.path.join(os.path.dirname(here), "oracle")]
+    out = subprocess.run([sys.executable, "-c", _RETRY.format(path=path, so=str(so))], capture_output=True, text=True,
+                         timeout=100)
+    assert out.returncode == 0 and "RETRY_OK" in out.stdout, out.stdout + out.stderr
