@@ -415,6 +415,34 @@ SFV_DEV void pair_slot(const DiffArgs &a, const double *A, int code, double ivol
   }
 }
 
+// With a viscosity per cell the reduced rows of a sub-element with a derived face
+// are symmetric in energy only where its stored faces are perpendicular to that
+// face (n its unit normal, t = tr(H) over the stored faces, H_2 the part of H
+// across n, r the row of H along it): their form is then
+//   mu0 (|H|^2 + tr(H)^2 / 3) + (mu - mu0) (2 |sym H_2|^2 - t^2 / 2 + |r|^2) > 0.
+// Elsewhere a pivot can vanish in a well-conditioned system (a skewed fan of three
+// prisms with viscosities 8 : 1), so such vertices are pivoted.  On extruded meshes
+// the faces are perpendicular to rounding.
+SFV_DEV bool skew_slot(const double *A, int code) {
+  double Ab[3] = {0, 0, 0};
+#pragma unroll
+  for (int e = 0; e < kSlotSrc; e++) {
+    const int b = (code >> (8 * e)) & 0xFF;
+    if (b != 0xFF && (b & kCodeDerived)) load3(A, b & kPosMask, 1.0, Ab);
+  }
+  bool skew = false;
+#pragma unroll
+  for (int e = 0; e < kSlotSrc; e++) {
+    const int b = (code >> (8 * e)) & 0xFF;
+    if (b & kCodeDerived) continue;  // the derived face or past the end of the list
+    double Ae[3];
+    load3(A, b & kPosMask, 1.0, Ae);
+    const double d = dot3(Ae, Ab);
+    skew = skew || !(d * d <= 1e-16 * dot3(Ae, Ae) * dot3(Ab, Ab));
+  }
+  return skew;
+}
+
 struct Group {
   const double *A;
   const int *ty, *sl, *scode;
@@ -573,10 +601,13 @@ __global__ __launch_bounds__(64) void k_visc(DiffArgs a) {
     form_rows(a, g, ni, lane, LPV, mu0, Lm, Lh);
     wsync_d();
     // uniform over the wavefront: the larger vertex's size, and pivoting where
-    // the matrix need not be symmetric positive definite
+    // the matrix need not be positive definite
     const int big = LPV == 32 ? max(ni, __shfl_xor(ni, 32)) : ni;
     const int nw = __builtin_amdgcn_readfirstlane(big);
-    const bool piv = a.pivot || __any(tag || (a.mu_cell && walls));
+    bool need = tag || (a.mu_cell && walls);
+    if (a.mu_cell)
+      for (int p = lane; p < ns; p += LPV) need = need || skew_slot(A, g.scode[p]);
+    const bool piv = a.pivot || __any(need);
     double *buf = L + o.buf;
     if (LPV == 32) {
       if (nw <= 4) momentum_inverse<12, LPV>(Lm, buf, ni, lane, piv);
@@ -1018,7 +1049,7 @@ __global__ __launch_bounds__(256) void k_visc_tile(DiffArgs a) {
   __shared__ int ty[kDiffMaxSub], sl[2 * kDiffMaxSub], sc[kDiffMaxSub];
   __shared__ double col[2][16 * T], rw[2][16 * T];
   __shared__ int prow[16 * T], inv[16 * T];
-  __shared__ int any_wall;
+  __shared__ int any_piv;
   const DevMesh &m = a.m;
   const long v = blockIdx.x;
   const int tid = threadIdx.x;
@@ -1029,7 +1060,7 @@ __global__ __launch_bounds__(256) void k_visc_tile(DiffArgs a) {
   const bool tag = dd >> 56 & 1, sym = !tag && !a.mu_cell;
   double *const pre = a.pre + (dd & 0xFFFFFFFFFFFFull);
   const double mu0 = a.mu_cell ? *a.mu_min : a.p.mu0;
-  if (tid == 0) any_wall = 0;
+  if (tid == 0) any_piv = 0;
   if (tid < 2 * kDiffMaxSub) sl[tid] = -1;
   __syncthreads();
   if (tid < nf) {
@@ -1039,7 +1070,7 @@ __global__ __launch_bounds__(256) void k_visc_tile(DiffArgs a) {
     for (int d = 0; d < 3; d++) A[3 * pos + d] = m.sfn[d * m.SF + s] * ar;
     if (pos < ni) {
       ty[pos] = face_type(a, fp, s);
-      if (fp & kPosBound) any_wall = 1;
+      if (a.mu_cell && (fp & kPosBound)) any_piv = 1;
     }
   }
   if (tid < ns) {
@@ -1054,7 +1085,9 @@ __global__ __launch_bounds__(256) void k_visc_tile(DiffArgs a) {
     }
   }
   __syncthreads();
-  const bool piv = a.pivot || tag || (a.mu_cell && any_wall);
+  if (a.mu_cell && tid < ns && skew_slot(A, sc[tid])) any_piv = 1;
+  __syncthreads();
+  const bool piv = a.pivot || tag || any_piv;
   const int ri = tid & 15, cj = tid >> 4;
   // entry (l, po) of a system: the sub-elements the two faces share
   auto shared_slots = [&](int l, int po, int side) -> int {
