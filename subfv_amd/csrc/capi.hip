@@ -328,6 +328,9 @@ std::string pack_groups(const subfv::HostMesh &hm, const std::vector<int> &off, 
       v++;
     if (v == vb) return "vertex " + std::to_string(v + 1) + " has more than " + std::to_string(kGrpSub) +
                         " sub-faces or " + std::to_string(kGrpSlots) + " sub-elements";
+    // vertices of no element: nothing to sweep, and no sub-face that the group's
+    // spare threads could load
+    if (off[v] == sf0) continue;
     const int hdr[kGrpHdr] = {vb, v - vb, sf0, off[v] - sf0, se0, hm.v_seoff[v] - se0, 0, 0};
     grp.insert(grp.end(), hdr, hdr + kGrpHdr);
     for (int u = vb; u < v; u++)
@@ -1599,6 +1602,8 @@ int subfv_compute_rhs_lagrange(subfv_ctx *c, const double *sol, const double *ma
   a.mass = dmass;
   a.T = T;
   a.vp = dvp;
+  // NaN (0 / 0 of an empty nodal system) at the vertices of no element that lie in no group
+  HIPCHK(c, hipMemsetAsync(dvp, 0xFF, 3 * m.V * sizeof(double), s));
   a.b2d = b2d ? 1 : 0;
   a.nblocks = m.ngroups;
   a.per_xcd = (m.ngroups + 7) / 8;

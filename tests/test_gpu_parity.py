@@ -9,7 +9,7 @@ import pytest
 
 import oracle as O
 from subfv_amd import meshgen as mg
-from subfv_amd.api import Solver, SubfvError, make_config
+from subfv_amd.api import HostMesh, Solver, SubfvError, make_config
 
 pytestmark = pytest.mark.gpu
 
@@ -292,3 +292,34 @@ def test_arrays_longer_than_a_rearranged_piece_bit_exact(solver):
     other = rhs[::-1].copy()
     solver.put("rhs", other)
     assert np.array_equal(solver.get("rhs"), other)
+
+
+@pytest.mark.parametrize("spare", [1, 64, 65, 400])
+@pytest.mark.parametrize("device", [False, True])
+def test_vertices_without_elements_bit_exact(solver, spare, device):
+    """A mesh with vertices that no element uses (a msh file's geometry
+    points): numbered last, more than a vertex group holds of them."""
+    print(f"[gpu] spare vertices {spare} device={device}", flush=True)
+    mesh = mg.tri_mesh(6)
+    rng = np.random.default_rng(spare)
+    mesh.coord = np.concatenate([mesh.coord, rng.random((spare, 3))])
+    if device:
+        solver.build_mesh(mesh)
+    else:
+        solver.upload_mesh(HostMesh(mesh), mesh.boundary_2d)
+    om = O.OracleMesh(mesh)
+    sol = mg.vortex_state(om.elem_coord)
+    for second in (False, True):
+        kw = dict(second_order=second, cfl=0.4)
+        solver.set_config(make_config("multi_point", **kw))
+        rhs, sl, vp = solver.compute_euler_flux(sol, want_vp=True)
+        r_rhs, r_sl, r_vp = om.compute_euler_flux(O.make_config("multi_point", **kw), sol, want_vp=True)
+        assert np.array_equal(rhs, r_rhs) and np.array_equal(sl, r_sl) and np.array_equal(vp, r_vp)
+        solver.set_time(0.0)
+        solver.put_sol(sol)
+        solver.run(3, 0)
+        st, ref, _ = om.run(O.make_config("multi_point", **kw), sol, 3, 0)
+        assert st == 0 and np.array_equal(solver.get_sol(), ref)
+    mass = 0.5 + rng.random(om.n_elems)
+    for got, want in zip(solver.compute_rhs_lagrange(sol, mass), om.compute_rhs_lagrange(sol, mass)):
+        assert np.array_equal(got, want, equal_nan=True)
