@@ -194,7 +194,8 @@ struct UpdateArgs {
   double *Uout;       // [C][5]
   const double *rhs, *rhs2, *sl;
   const double *diag; // [C][25] column-major 5x5 blocks (kDiagFull)
-  const double *Ud, *dblk;  // the residual's state and the cells' viscous blocks (kDiagBlocks)
+  const double *Ud;   // the residual's state (flux limiting, kDiagBlocks)
+  const double *dblk; // the cells' viscous blocks (kDiagBlocks)
   double cv;
   const double *rdiff;// [C][4] viscous rhs of components 2..5 (added after flux limiting), or null
   double *W;          // [C][6] primitives and sound speed of Uout (as k_prim), or null
@@ -230,11 +231,13 @@ SFV_DEV double stage_cell(const UpdateArgs &a, const StepDt &st, const double *U
   const double vol = a.m.cvol[c];
   const double lam = a.sl[c];
   if (a.flux_limit) {
+    // about the state of the residual, which is not the stage's in the second
+    // half of the two-stage loop (ns_main.F90:88-95)
     double r2[5], x[5], y[5];
     double cf = vol / st.dt_fl + lam;
     for (int k = 0; k < 5; k++) {
       r2[k] = a.rhs2[k * C + c];
-      x[k] = u[k] + r[k] / cf;
+      x[k] = (a.Ud == U ? u[k] : a.Ud[5 * c + k]) + r[k] / cf;
       y[k] = (r2[k] - r[k]) / cf;
     }
     double om = max_omega_pos(x, y);
