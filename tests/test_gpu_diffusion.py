@@ -263,6 +263,34 @@ def test_largest_vertex_last_matches_oracle(solver, k, rings, law):
     viscous_matches_oracle(solver, mesh, law, *TAGGED)
 
 
+def mixed_tags(x):
+    """untagged, Dirichlet and Neumann velocities (both with Dirichlet
+    temperatures) in turn over the boundary"""
+    return int(np.floor(7.3 * x[0] + 5.1 * x[1] + 3.7 * x[2])) % 3
+
+
+# tagged vertices outside the 32-lane class: 64 lanes (hexahedra; a fan between
+# two layers, with 11 and more stored faces) and a workgroup per vertex (tets)
+@pytest.mark.parametrize("law", ["constant", "sutherland"])
+@pytest.mark.parametrize("mk", [lambda: mg.hex_mesh(3), lambda: fan_prism_mesh(7, 2), lambda: fan_prism_mesh(12, 1),
+                                lambda: mg.tet_mesh(3), lambda: fan_prism_mesh(16, 2)],
+                         ids=["hex3", "fan7x2", "fan12", "tet3", "fan16x2"])
+def test_tagged_boundaries_of_each_class_match_oracle(solver, mk, law):
+    mesh = tag_boundary(mk(), mixed_tags)
+    print(f"[gpu] viscous tagged {mesh.name} {mesh.n_elems} {law}", flush=True)
+    assert set(np.unique(mesh.bf_tag)) == {1, 2}
+    viscous_matches_oracle(solver, mesh, law, *TAGGED)
+
+
+@pytest.mark.parametrize("law", ["constant", "sutherland"])
+def test_viscous_terms_beside_spare_vertices_match_oracle(solver, law):
+    """Vertices of no element, numbered last: no faces, no slots."""
+    print(f"[gpu] viscous spare vertices {law}", flush=True)
+    mesh = mg.tri_mesh(6)
+    mesh.coord = np.concatenate([mesh.coord, np.random.default_rng(2).random((70, 3))])
+    viscous_matches_oracle(solver, mesh, law, {}, {})
+
+
 def skew_fan_mesh(k, seed, amp):
     """k prisms around an axis in one layer, every vertex displaced: the wall
     faces are not perpendicular to the faces between the prisms."""

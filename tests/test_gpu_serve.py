@@ -5,6 +5,7 @@ instance's arithmetic is that of subfv_run)."""
 import numpy as np
 import pytest
 
+import oracle as O
 from subfv_amd import meshgen as mg
 from subfv_amd import serve as S
 from subfv_amd.api import Solver
@@ -199,3 +200,37 @@ def test_admission_estimate_covers_what_an_instance_holds(mk):
         batch.close()
         s.close()
     assert held <= S.device_bytes(r) <= 1.4 * held + (4 << 20)
+
+
+@pytest.mark.parametrize("mode", [0, 1, 2])
+def test_shortened_updates_in_a_batch_match_oracle(mode):
+    """Members whose first updates are shortened (0 < omega < 1), beside one
+    that is not: the oracle's bits after the run goes on."""
+    print(f"[gpu] batch shortened updates mode={mode}", flush=True)
+    meshes = [mg.quad_mesh(12), mg.tri_mesh(9), mg.quad_mesh(40)]
+    speeds = [2.0, 2.0, 0.0]
+    solvers, batch = [S.Solver(0) for _ in meshes], S.Batch(0)
+    try:
+        sols = []
+        for s, mesh, u in zip(solvers, meshes, speeds):
+            s.upload_mesh(S.HostMesh(mesh), mesh.boundary_2d)
+            s.set_config(S.make_config("multi_point", cfl=8.0 if u else 0.4))
+            s.set_time(0.0)
+            sols.append(mg.init_1drp(s.elem_coord, 0.5, [1, -u, 0, 0, 0.4], [1, u, 0, 0, 0.4]))
+            s.put_sol(sols[-1])
+        batch.run(solvers, 5, mode)
+        batch.wait()
+        for s, mesh, u, sol in zip(solvers, meshes, speeds, sols):
+            om = O.OracleMesh(mesh)
+            cfg = O.make_config("multi_point", cfl=8.0 if u else 0.4)
+            r, sl = om.compute_euler_flux(cfg, sol)
+            omega = om.add_timedisc_and_solve(cfg, sol, r, sl, 1.0, 1.0, cfg.cfl, 0.0)["omega"]
+            assert 1e-6 < omega < 1.0 if u else omega == 1.0
+            st, ref, info = om.run(cfg, sol, 5, 0)
+            assert st == 0
+            t, _ = s.run(0, 0)
+            assert np.array_equal(s.get_sol(), ref) and t == info["t"]
+    finally:
+        batch.close()
+        for s in solvers:
+            s.close()
