@@ -670,11 +670,12 @@ int launch_grad(subfv_ctx *c, const double *U, int method, const double *W = nul
 template <int DIAG>
 void launch_update_d(subfv_ctx *c, const UpdateArgs &u, bool fold) {
   dim3 g(u.nblk), b(kCellThreads);
-  if (fold) {
-    hipLaunchKernelGGL((k_update<DIAG, true>), g, b, 0, c->stream, u);
-    hipLaunchKernelGGL(k_finish<DIAG>, g, b, 0, c->stream, u);
-    return;
-  }
+  if constexpr (DIAG != kDiagFull)  // the single update, which never folds
+    if (fold) {
+      hipLaunchKernelGGL((k_update<DIAG, true>), g, b, 0, c->stream, u);
+      hipLaunchKernelGGL(k_finish<DIAG>, g, b, 0, c->stream, u);
+      return;
+    }
   hipLaunchKernelGGL((k_update<DIAG, false>), g, b, 0, c->stream, u);
   hipLaunchKernelGGL(k_finalize_omega, dim3(1), b, 0, c->stream, (const double *)c->oblk, (int)g.x, c->st, u.advance_t);
   hipLaunchKernelGGL(k_update_fixup<DIAG>, g, b, 0, c->stream, u);

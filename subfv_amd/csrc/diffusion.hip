@@ -239,8 +239,7 @@ SFV_DEV void stress(const double H[3][3], double c1, double c2, double c3, doubl
 }
 
 // g_l = column of S(l, p) V (f = 0) or S(l, p) e_f (f > 0) for the slot's
-// stored faces; gh the heat system's.  FORM: a viscosity per cell.
-template <bool FORM>
+// stored faces; gh the heat system's.
 SFV_DEV void slot_fluxes(const double *A, const int *ty, int f, SlotReg &r) {
   double H[3][3], S[3][3], Sn[3][3];
   for (int i = 0; i < 3; i++) {
@@ -250,7 +249,7 @@ SFV_DEV void slot_fluxes(const double *A, const int *ty, int f, SlotReg &r) {
   if (r.posb >= 0) add_derived(H, r.Ab, r.ia2);
   stress(H, r.mu, r.c2, r.c3, r.ivol, S);
   // boundary rows take the constant-viscosity form, scaled by the cell's mu
-  if (FORM) stress(H, r.mu, 0.0, r.mu / 3.0, r.ivol, Sn);
+  stress(H, r.mu, 0.0, r.mu / 3.0, r.ivol, Sn);
   double q[3];
   const double qb = r.posb >= 0 ? dot3(r.Ab, r.Q) * r.ia2 : 0.0;
   for (int d = 0; d < 3; d++) q[d] = r.kv * (r.Q[d] - r.Ab[d] * qb);
@@ -264,7 +263,7 @@ SFV_DEV void slot_fluxes(const double *A, const int *ty, int f, SlotReg &r) {
       load3(A, pos, b & kCodeRight ? -1.0 : 1.0, Ae);
       for (int i = 0; i < 3; i++) {
         double x = dot3(S[i], Ae);
-        if (FORM && (t & kTyV) == 1) x = dot3(Sn[i], Ae);
+        if ((t & kTyV) == 1) x = dot3(Sn[i], Ae);
         r.g[e][i] = (t & kTyV) == 2 ? 0.0 : x;
       }
       r.gh[e] = (t >> kTyTShift & 3) == 2 ? 0.0 : tf * dot3(q, Ae);
@@ -646,7 +645,7 @@ __global__ __launch_bounds__(64) void k_visc(DiffArgs a) {
   for (int t = lane; t < 4 * ns; t += LPV) {
     slot_load<true>(a, se0 + (t >> 2), r, mu0);
     slot_faces(A, r);
-    slot_fluxes<FORM || MODE == kGlobal>(A, ty, t & 3, r);
+    slot_fluxes(A, ty, t & 3, r);
     if ((t & 3) == 0)
 #pragma unroll
       for (int e = 0; e < kSlotSrc; e++)
@@ -694,7 +693,7 @@ __global__ __launch_bounds__(64) void k_visc(DiffArgs a) {
     if (rounds > 1) {
       slot_load<true>(a, se0 + (t >> 2), r, mu0);
       slot_faces(A, r);
-      slot_fluxes<FORM || MODE == kGlobal>(A, ty, f, r);
+      slot_fluxes(A, ty, f, r);
     }
     double H[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}}, h[3] = {0, 0, 0};
 #pragma unroll
@@ -1148,7 +1147,7 @@ __global__ __launch_bounds__(256) void k_visc_tile(DiffArgs a) {
     __syncthreads();
   }
   {  // heat: at most 64 unknowns
-    constexpr int TH = T < 4 ? T : 4;
+    constexpr int TH = 4;
     double x[TH][TH];
 #pragma unroll
     for (int i = 0; i < TH; i++)
@@ -1288,9 +1287,7 @@ static hipError_t launch_gather(DiffArgs a, int rhs, int blocks, hipStream_t s) 
 static hipError_t launch_tile(DiffArgs a, hipStream_t s) {
   const int n = 3 * a.nim;
   const dim3 g((unsigned)a.m.V), b(256);
-  if (n <= 64)
-    hipLaunchKernelGGL(k_visc_tile<4>, g, b, 0, s, a);
-  else if (n <= 112)
+  if (n <= 112)
     hipLaunchKernelGGL(k_visc_tile<7>, g, b, 0, s, a);
   else
     hipLaunchKernelGGL(k_visc_tile<12>, g, b, 0, s, a);

@@ -135,7 +135,7 @@ __global__ __launch_bounds__(kCellThreads) void k_init_1drp(DevMesh m, Init1drp 
 
 struct GatherArgs {
   DevMesh m;
-  const double *P;   // first-order partials [SE][6], node-sorted slots
+  const double *P;   // first-order partials [SE][kSlotStride], node-sorted slots
   const double *P2;  // second-order partials or null
   double *rhs;       // [5][C]
   double *rhs2;      // [5][C] (second order)

@@ -26,9 +26,9 @@
 // registers: 1,035, 150 and 29.2 us.
 //
 // Output: one row of six partial sums per node-sorted sub-element slot q
-// (vertex-major, so a group's rows are one contiguous run): P[6*q + k] = sum
-// over the vertex's sub-faces of area*flux_k (k < 5) and P[6*q + 5] = sum of
-// area*max(0, -s).  Thread q of the group owns slot q; its contributors (the
+// (vertex-major, so a group's rows are one contiguous run), kSlotStride doubles
+// apart: P[kSlotStride*q + k] = sum over the vertex's sub-faces of area*flux_k
+// (k < 5) and P[kSlotStride*q + 5] = sum of area*max(0, -s).  Thread q of the group owns slot q; its contributors (the
 // group-local sub-faces touching the slot's cell, in increasing order) come
 // from the static table se_src.
 #pragma once
@@ -43,7 +43,7 @@ struct FluxArgs {
   const double *U;      // [C][5] conservative state, sol(5, n_elems)
   const double *G;      // [C][15] cell gradients, 3*k + d fastest (second order)
   const double *W;      // [C][6] primitives and sound speed of U (k_prim), or null
-  double *P;            // [SE][6] node-sorted slots
+  double *P;            // [SE][kSlotStride] node-sorted slots
   double *vp;           // [3][V] nodal velocity output or null
   int *err;
   const double *t;      // physical time (time-dependent BCs)
