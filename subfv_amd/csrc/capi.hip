@@ -803,9 +803,9 @@ int diffusion_buffers(subfv_ctx *c) {
   std::vector<uint64_t> off(h.nv);
   uint64_t at = 0;
   for (int v = 0; v < h.nv; v++) {
-    const uint64_t ni = st[v] & 0xFF, tag = st[v] >> 8;
+    const uint64_t ni = st[v] & 0xFF, tag = st[v] >> 8 & 1, skew = st[v] >> 9;
     const uint64_t nb = tag || c->diff_cls == kDiffLarge ? ni * ni : ni * (ni + 1) / 2;
-    off[v] = at | ni << 48 | tag << 56;
+    off[v] = at | ni << 48 | tag << 56 | skew << 57;
     at += 10 * nb;
   }
   c->diff_lds = c->diff_cls == kDiffLarge ? 0 : apply_lds_wave(h.nv, kDiffApplyVerts[c->diff_cls], [&](long v) {

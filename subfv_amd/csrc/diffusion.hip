@@ -56,7 +56,16 @@ SFV_DEV void wsync_d() {
 SFV_DEV int tri(int k) { return k * (k + 1) / 2; }
 
 // One thread per vertex: which faces are derived, every face's place and
-// every slot's code; once per mesh.
+// every slot's code; once per mesh.  vstat: stored faces, << 8 tagged, << 9 skewed.
+//
+// Skewed: a stored face is not perpendicular to its sub-element's derived one.
+// With a viscosity per cell the reduced rows are positive definite only where it
+// is (t = tr(H) over the stored faces, H_2 the part of H across the derived face's
+// normal, r the row of H along it): the sub-element's form is then
+//   mu0 (|H|^2 + tr(H)^2 / 3) + (mu - mu0) (2 |sym H_2|^2 - t^2 / 2 + |r|^2) > 0.
+// Elsewhere a pivot can vanish in a well-conditioned system (a skewed fan of three
+// prisms with viscosities 8 : 1), so such vertices are pivoted then.  On extruded
+// meshes the faces are perpendicular to rounding.
 __global__ __launch_bounds__(256) void k_diff_tables(DevMesh m, int *vstat, uint8_t *fpos, uint32_t *scode,
                                                      double *sivol) {
   const long v = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -64,6 +73,7 @@ __global__ __launch_bounds__(256) void k_diff_tables(DevMesh m, int *vstat, uint
   const int sf0 = m.sf_off[v], nf = m.sf_off[v + 1] - sf0;
   const int se0 = m.se_off[v], se1 = m.se_off[v + 1];
   uint64_t der = 0;
+  int skew = 0;
   for (int q = se0; q < se1; q++) {
     const int se = m.v_seid[q];
     sivol[q] = 1.0 / m.se_vol[se];
@@ -73,7 +83,14 @@ __global__ __launch_bounds__(256) void k_diff_tables(DevMesh m, int *vstat, uint
         walls++;
         l = m.se_sf[p] - sf0;
       }
-    if (walls == 1) der |= 1ull << l;
+    if (walls == 1) {
+      der |= 1ull << l;
+      for (int p = m.se_sfoff[se]; p < m.se_sfoff[se + 1]; p++) {
+        double d = 0.0;
+        for (int k = 0; k < 3; k++) d += m.sfn[k * m.SF + m.se_sf[p]] * m.sfn[k * m.SF + sf0 + l];
+        if (m.se_sf[p] != sf0 + l && !(fabs(d) <= 1e-8)) skew = 1;
+      }
+    }
   }
   const int nd = __popcll(der), ni = nf - nd;
   int tag = 0;
@@ -101,7 +118,7 @@ __global__ __launch_bounds__(256) void k_diff_tables(DevMesh m, int *vstat, uint
       }
     scode[q] = code;
   }
-  vstat[v] = ni | tag << 8;
+  vstat[v] = ni | tag << 8 | skew << 9;
 }
 
 // ------------------------------------------------------------- LDS layout
@@ -414,34 +431,6 @@ SFV_DEV void pair_slot(const DiffArgs &a, const double *A, int code, double ivol
   }
 }
 
-// With a viscosity per cell the reduced rows of a sub-element with a derived face
-// are symmetric in energy only where its stored faces are perpendicular to that
-// face (n its unit normal, t = tr(H) over the stored faces, H_2 the part of H
-// across n, r the row of H along it): their form is then
-//   mu0 (|H|^2 + tr(H)^2 / 3) + (mu - mu0) (2 |sym H_2|^2 - t^2 / 2 + |r|^2) > 0.
-// Elsewhere a pivot can vanish in a well-conditioned system (a skewed fan of three
-// prisms with viscosities 8 : 1), so such vertices are pivoted.  On extruded meshes
-// the faces are perpendicular to rounding.
-SFV_DEV bool skew_slot(const double *A, int code) {
-  double Ab[3] = {0, 0, 0};
-#pragma unroll
-  for (int e = 0; e < kSlotSrc; e++) {
-    const int b = (code >> (8 * e)) & 0xFF;
-    if (b != 0xFF && (b & kCodeDerived)) load3(A, b & kPosMask, 1.0, Ab);
-  }
-  bool skew = false;
-#pragma unroll
-  for (int e = 0; e < kSlotSrc; e++) {
-    const int b = (code >> (8 * e)) & 0xFF;
-    if (b & kCodeDerived) continue;  // the derived face or past the end of the list
-    double Ae[3];
-    load3(A, b & kPosMask, 1.0, Ae);
-    const double d = dot3(Ae, Ab);
-    skew = skew || !(d * d <= 1e-16 * dot3(Ae, Ae) * dot3(Ab, Ab));
-  }
-  return skew;
-}
-
 struct Group {
   const double *A;
   const int *ty, *sl, *scode;
@@ -557,7 +546,7 @@ __global__ __launch_bounds__(64) void k_visc(DiffArgs a) {
   const int se0 = m.se_off[v], ns = m.se_off[v + 1] - se0;
   const uint64_t dd = a.doff[v];
   const int ni = (int)(dd >> 48 & 0xFF);
-  const bool tag = dd >> 56 & 1;
+  const bool tag = dd >> 56 & 1, skew = dd >> 57 & 1;
   double *const pre = a.pre + (dd & 0xFFFFFFFFFFFFull);
   const bool sym = MODE == kGlobal && !tag && !a.mu_cell;  // formed here: all blocks, in LDS
   const double mu0 = a.mu_cell ? *a.mu_min : a.p.mu0;
@@ -603,10 +592,7 @@ __global__ __launch_bounds__(64) void k_visc(DiffArgs a) {
     // the matrix need not be positive definite
     const int big = LPV == 32 ? max(ni, __shfl_xor(ni, 32)) : ni;
     const int nw = __builtin_amdgcn_readfirstlane(big);
-    bool need = tag || (a.mu_cell && walls);
-    if (a.mu_cell)
-      for (int p = lane; p < ns; p += LPV) need = need || skew_slot(A, g.scode[p]);
-    const bool piv = a.pivot || __any(need);
+    const bool piv = a.pivot || __any(tag || (a.mu_cell && (walls || skew)));
     double *buf = L + o.buf;
     if (LPV == 32) {
       if (nw <= 4) momentum_inverse<12, LPV>(Lm, buf, ni, lane, piv);
@@ -1048,7 +1034,7 @@ __global__ __launch_bounds__(256) void k_visc_tile(DiffArgs a) {
   __shared__ int ty[kDiffMaxSub], sl[2 * kDiffMaxSub], sc[kDiffMaxSub];
   __shared__ double col[2][16 * T], rw[2][16 * T];
   __shared__ int prow[16 * T], inv[16 * T];
-  __shared__ int any_piv;
+  __shared__ int any_wall;
   const DevMesh &m = a.m;
   const long v = blockIdx.x;
   const int tid = threadIdx.x;
@@ -1059,7 +1045,7 @@ __global__ __launch_bounds__(256) void k_visc_tile(DiffArgs a) {
   const bool tag = dd >> 56 & 1, sym = !tag && !a.mu_cell;
   double *const pre = a.pre + (dd & 0xFFFFFFFFFFFFull);
   const double mu0 = a.mu_cell ? *a.mu_min : a.p.mu0;
-  if (tid == 0) any_piv = 0;
+  if (tid == 0) any_wall = 0;
   if (tid < 2 * kDiffMaxSub) sl[tid] = -1;
   __syncthreads();
   if (tid < nf) {
@@ -1069,7 +1055,7 @@ __global__ __launch_bounds__(256) void k_visc_tile(DiffArgs a) {
     for (int d = 0; d < 3; d++) A[3 * pos + d] = m.sfn[d * m.SF + s] * ar;
     if (pos < ni) {
       ty[pos] = face_type(a, fp, s);
-      if (a.mu_cell && (fp & kPosBound)) any_piv = 1;
+      if (fp & kPosBound) any_wall = 1;
     }
   }
   if (tid < ns) {
@@ -1084,9 +1070,7 @@ __global__ __launch_bounds__(256) void k_visc_tile(DiffArgs a) {
     }
   }
   __syncthreads();
-  if (a.mu_cell && tid < ns && skew_slot(A, sc[tid])) any_piv = 1;
-  __syncthreads();
-  const bool piv = a.pivot || tag || any_piv;
+  const bool piv = a.pivot || tag || (a.mu_cell && (any_wall || (dd >> 57 & 1)));
   const int ri = tid & 15, cj = tid >> 4;
   // entry (l, po) of a system: the sub-elements the two faces share
   auto shared_slots = [&](int l, int po, int side) -> int {

@@ -35,7 +35,7 @@ enum DiffClass : int { kDiffHalf = 0, kDiffWave = 1, kDiffLarge = 2 };
 struct DiffArgs {
   DevMesh m;
   DiffParams p;
-  const uint64_t *doff;    // [V] offset of the vertex's inverses, stored faces << 48, tagged << 56
+  const uint64_t *doff;    // [V] offset of the vertex's inverses, stored faces << 48, tagged << 56, skewed << 57
   double *pre;             // inverses of the nodal systems
   const double *U;         // [C][5]
   double *PD;              // [SE][kDiffSlot or kDiffRow] node-sorted slot partials
