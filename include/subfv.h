@@ -150,9 +150,8 @@ int subfv_set_config(subfv_ctx *ctx, const subfv_config *cfg);
  * per-subface flux and nodal-solver kernel).  SUBFV_ARITH_EXACT (the default)
  * evaluates the reference's expressions as written, bit-identical to it;
  * SUBFV_ARITH_FAST compiles it with products contracted into fused
- * multiply-adds and divisions evaluated as products with reciprocals (one
- * reciprocal where a divisor repeats, as across the nodal-solver
- * iterations): results within 1e-12 relative of the reference's after 200
+ * multiply-adds and most divisions evaluated as products with reciprocals
+ * (where a divisor repeats, both forms share a refined one): results within 1e-12 relative of the reference's after 200
  * steps (tested), not bit-identical.  Every other kernel stays exact. */
 #define SUBFV_ARITH_EXACT 0
 #define SUBFV_ARITH_FAST 1
