@@ -282,6 +282,29 @@ def test_tagged_boundaries_of_each_class_match_oracle(solver, mk, law):
     viscous_matches_oracle(solver, mesh, law, *TAGGED)
 
 
+def pyramid_mesh(n, seed=3):
+    """n^3 hexahedra, each split into six pyramids about a displaced centre:
+    four sub-faces of a cell meet at its apex."""
+    h = mg.hex_mesh(n)
+    v = h.elem_vert.reshape(-1, 8)
+    rng = np.random.default_rng(seed)
+    centre = h.coord[v - 1].mean(axis=1) + 0.05 / n * rng.uniform(-1, 1, (len(v), 3))
+    ids = h.n_vert + 1 + np.arange(len(v))
+    faces = ([0, 1, 2, 3], [4, 7, 6, 5], [0, 4, 5, 1], [1, 5, 6, 2], [2, 6, 7, 3], [3, 7, 4, 0])
+    ev = np.concatenate([np.column_stack([v[:, f], ids]) for f in faces])
+    return mg.Mesh(np.concatenate([h.coord, centre]), np.full(len(ev), 7, np.int32), ev.astype(np.int32).ravel(),
+                   boundary_2d=False, name="pyramid")
+
+
+# the 64-lane class (12 stored faces at the apex) and the large one (36 faces at
+# an inner corner)
+@pytest.mark.parametrize("law", ["constant", "sutherland"])
+@pytest.mark.parametrize("n", [1, 2])
+def test_pyramids_match_oracle(solver, n, law):
+    print(f"[gpu] viscous pyramids {n} {law}", flush=True)
+    viscous_matches_oracle(solver, pyramid_mesh(n), law, dict(boundary_2d=False), {})
+
+
 @pytest.mark.parametrize("law", ["constant", "sutherland"])
 def test_viscous_terms_beside_spare_vertices_match_oracle(solver, law):
     """Vertices of no element, numbered last: no faces, no slots."""
